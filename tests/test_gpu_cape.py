@@ -611,3 +611,22 @@ def test_warm_parts_match_one_launch(hip, monkeypatch):
             else:
                 np.testing.assert_array_equal(a, b)
     assert got[0][-1]['columns'] == 3000
+
+
+@pytest.mark.parametrize('adiabat', [1, 2, 3, 4])
+@pytest.mark.parametrize('ncol,nk', [(1, 60), (63, 40), (1024, 40), (1025, 33), (2111, 40),
+                                     (65537, 24), (131072, 20), (131073, 20)])
+def test_small_launches_match_the_large_loop(hip, adiabat, ncol, nk):
+    """Plain launches of at most two waves per SIMD spread their columns over
+    the waves and iterate with a loop of their own; counted launches always
+    take the large grids' loop.  Same columns, same bits, on both sides of the
+    limit and with a partly filled last wave."""
+    import torch
+    c = synthetic.sigma_columns_torch(ncol, nk, 7 * ncol + adiabat)
+    args = [c[k] for k in ('p', 't', 'td', 'ps', 'ts', 'tds')]
+    kw = dict(pinc=500., source=1 + adiabat % 3, adiabat=adiabat)
+    small = hip.cape(*args, **kw)
+    large = hip.cape(*args, stats=True, **kw)
+    for a, b in zip(small, large[:4]):
+        assert torch.equal(a, b)
+    assert large[4]['columns'] == ncol

@@ -160,94 +160,155 @@ XC_HD __forceinline__ void fp_eval_ops(T p2, T pi2, T logp, T t1, T th1, T qv1, 
 
 #if defined(__HIP_DEVICE_COMPILE__)
 // The accurate mode's evaluation on the device: the operations of
-// fp_eval_ops in the same order, with the raw IEEE division kernels and
-// exp_core (phys.h).  Wherever those give the library's values -- every
-// operand in the normal range, exp arguments within (-87, 88) -- the result
-// is fp_eval_ops<float, MATH_LIB>'s bit for bit; a zero or infinite divisor
-// or other special value turns the raw division into NaN, which reaches th2
-// (every quotient feeds qv2 or the exponent), and the evaluation is then
-// repeated with the library's operations.  Divisors: the ice ramp's
-// 273.15 - 233.15 by a correctly rounded reciprocal; the two latent-heat
-// terms share one reciprocal of cpm * tbar.
-template <bool ICE>
+// fp_eval_ops in the same order, with the raw IEEE division kernels,
+// exp_core and exp_small (phys.h).  Wherever those give the library's values
+// -- every operand in the normal range, exp arguments within (-87, 88), the
+// last one within EXP_SMALL_MAX (a sub-step that changes theta by less than
+// 1.4 times) -- the result is fp_eval_ops<float, MATH_LIB>'s bit for bit; a
+// zero or infinite divisor or other special value turns the raw division into
+// NaN, which reaches `arg` (every quotient feeds qv2 or the exponent).  The
+// caller repeats the work with the library's operations where
+// !(|arg| < EXP_SMALL_MAX).  Divisors: the ice ramp's 273.15 - 233.15 by a
+// correctly rounded reciprocal; the two latent-heat terms share one
+// reciprocal of cpm * tbar.
+//
+// The reference's means (tbar, qvbar, ..) carry factors 0.5, which are exact:
+// they are folded into the constants (and the latent heat and cpm * tbar kept
+// doubled), so every other operation rounds as the reference's does.
+//
+// REGIME: the phases an ice adiabat's evaluation has to consider.  REG_MIXED
+// is the general one.  With fliq = 1 (REG_LIQUID) the ice saturation enters
+// as a zero times a finite number, and for a pseudo-adiabat the ice terms are
+// the constant zero; with fliq = 0 (REG_ICE) likewise the liquid ones.  The
+// results are REG_MIXED's bit for bit; regime_hot and regime_cold say when a
+// parcel's evaluation may use them.
+enum { REG_MIXED = 0, REG_LIQUID = 1, REG_ICE = 2 };
+
+// fliq = 1 exactly, and the ice saturation mixing ratio finite: esi(310 K) is
+// 8794 Pa
+__device__ __forceinline__ bool regime_hot(float p2, float t2)
+{
+    return t2 >= 273.15f && t2 < 310.0f && p2 > 10000.0f;
+}
+// fliq = 0 exactly, and the liquid saturation mixing ratio finite:
+// esl(233.15 K) is 19 Pa, and its exponent at 100 K is -43.5
+__device__ __forceinline__ bool regime_cold(float p2, float t2)
+{
+    return t2 <= 233.15f && t2 > 100.0f && p2 > 100.0f;
+}
+
+template <bool ICE, bool PSEUDO, int REGIME>
 __device__ __forceinline__ void fp_eval_raw(float p2, float pi2, float logp, float t1, float th1,
                                             float qv1, float ql1, float qi1, float qt,
                                             float thlast, float &th2, float &t2, float &qv2,
-                                            float &ql2, float &qi2)
+                                            float &ql2, float &qi2, float &arg)
 {
     using K = Phys<float>;
+    constexpr bool LIQ_ONLY = !ICE || REGIME == REG_LIQUID;
+    constexpr bool ICE_ONLY = ICE && REGIME == REG_ICE;
+    constexpr bool HAS_L = !(ICE_ONLY && PSEUDO), HAS_I = ICE && !(LIQ_ONLY && PSEUDO);
     constexpr float RAMP = 273.15f - 233.15f;
     constexpr float RRAMP = 1.0f / RAMP;
     t2 = thlast * pi2;
     const float tc = t2 - 273.15f;
-    const float esl = 611.2f * exp_core(div_raw(17.67f * tc, t2 - 29.65f));
-    const float qsl = div_raw(K::eps * esl, p2 - esl);
-    if (ICE) {
+    float qsl = 0.0f, qsi = 0.0f;
+    if (!ICE_ONLY) {
+        const float es = 611.2f * exp_core(div_raw(17.67f * tc, t2 - 29.65f));
+        qsl = div_raw(K::eps * es, p2 - es);
+    }
+    if (!LIQ_ONLY) {
+        const float es = 611.2f * exp_core(div_raw(21.8745584f * tc, t2 - 7.66f));
+        qsi = div_raw(K::eps * es, p2 - es);
+    }
+    if (LIQ_ONLY) {
+        qv2 = min_nan(qt, qsl);
+        qi2 = 0.0f;
+        ql2 = fmx(qt - qv2, 0.0f);
+    } else if (ICE_ONLY) {
+        qv2 = min_nan(qt, qsi);
+        qi2 = fmx(qt - qv2, 0.0f);
+        ql2 = 0.0f;
+    } else {
         const float fliq = fmx(fmn(div_const(t2 - 233.15f, RAMP, RRAMP), 1.0f), 0.0f);
         const float fice = 1.0f - fliq;
-        const float esi = 611.2f * exp_core(div_raw(21.8745584f * tc, t2 - 7.66f));
-        const float qsi = div_raw(K::eps * esi, p2 - esi);
-        qv2 = fmn(qt, fliq * qsl + fice * qsi);
+        qv2 = min_nan(qt, fliq * qsl + fice * qsi);
         qi2 = fmx(fice * (qt - qv2), 0.0f);
-    } else {
-        qv2 = fmn(qt, qsl);
-        qi2 = 0.0f;
+        ql2 = fmx(qt - qv2 - qi2, 0.0f);
     }
-    ql2 = fmx(qt - qv2 - qi2, 0.0f);
-    const float tbar = 0.5f * (t1 + t2);
-    const float qvbar = 0.5f * (qv1 + qv2);
-    const float qlbar = 0.5f * (ql1 + ql2);
-    const float lhv = K::lv1 - K::lv2 * tbar;
-    const float rm = K::rd + K::rv * qvbar;
-    float arg;
-    if (ICE) {
-        const float qibar = 0.5f * (qi1 + qi2);
-        const float lhs = K::ls1 - K::ls2 * tbar;
-        const float cpm = K::cp + K::cpv * qvbar + K::cpl * qlbar + K::cpi * qibar;
-        float a1, a2;
-        div2_raw(lhv * (ql2 - ql1), lhs * (qi2 - qi1), cpm * tbar, a1, a2);
-        arg = a1 + a2 + (div_raw(rm, cpm) - K::rddcp) * logp;
-    } else {
-        const float cpm = K::cp + K::cpv * qvbar + K::cpl * qlbar;
-        arg = div_raw(lhv * (ql2 - ql1), cpm * tbar) + (div_raw(rm, cpm) - K::rddcp) * logp;
+    const float tsum = t1 + t2;
+    const float qvsum = qv1 + qv2;
+    const float rm = K::rd + (0.5f * K::rv) * qvsum;
+    float cpm = K::cp + (0.5f * K::cpv) * qvsum;
+    if (HAS_L) cpm = cpm + (0.5f * K::cpl) * (ql1 + ql2);
+    if (HAS_I) cpm = cpm + (0.5f * K::cpi) * (qi1 + qi2);
+    const float den = cpm * tsum;
+    const float yden = rcp_rn(den);
+    arg = 0.0f;
+    if (HAS_L) arg = div_by((2.0f * K::lv1 - K::lv2 * tsum) * (ql2 - ql1), den, yden);
+    if (HAS_I) {
+        const float ai = div_by((2.0f * K::ls1 - K::ls2 * tsum) * (qi2 - qi1), den, yden);
+        arg = HAS_L ? arg + ai : ai;
     }
-    th2 = th1 * exp_core(arg);
+    arg = arg + (div_raw(rm, cpm) - K::rddcp) * logp;
+    th2 = th1 * exp_small(arg);
+}
+
+__device__ __forceinline__ bool arg_small(float arg)
+{
+    return __builtin_fabsf(arg) < EXP_SMALL_MAX;
 }
 #endif
 
-template <typename T, int MATH, bool ICE>
+// ln(p2 / p1) of a sub-step (:461).
+template <typename T, int MATH>
+XC_HD __forceinline__ T log_ratio(T p2, T p1)
+{
+    using F = Fn<T, MATH>;
+#if defined(__HIP_DEVICE_COMPILE__)
+    // the accurate mode's raw kernels, whose value is the library's bit for
+    // bit for a ratio within (1e-26, 1e26) of normal pressures; a zero,
+    // infinite, negative or NaN pressure fails the test
+    if constexpr (sizeof(T) == 4 && MATH == MATH_ACCURATE) {
+        const float l = log_core(div_raw(p2, p1));
+        if (__builtin_expect(__builtin_fabsf(l) < 60.0f, 1)) return l;
+    }
+#endif
+    return F::log(F::div(p2, p1));
+}
+
+template <typename T, int MATH, bool ICE, bool PSEUDO>
 XC_HD __forceinline__ void fp_eval(T p2, T pi2, T logp, T t1, T th1, T qv1, T ql1, T qi1,
                                    T qt, T thlast, T &th2, T &t2, T &qv2, T &ql2, T &qi2)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     if constexpr (sizeof(T) == 4 && MATH == MATH_ACCURATE) {
-        fp_eval_raw<ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast, th2, t2, qv2, ql2,
-                         qi2);
-        if (__builtin_expect(!__builtin_isfinite(th2), 0))
-            fp_eval_ops<T, MATH_LIB, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast,
-                                          th2, t2, qv2, ql2, qi2);
+        float arg;
+        fp_eval_raw<ICE, PSEUDO, REG_MIXED>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast,
+                                            th2, t2, qv2, ql2, qi2, arg);
+        if (__builtin_expect(!arg_small(arg), 0))
+            fp_eval_ops<T, MATH_LIB, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt,
+                                                  thlast, th2, t2, qv2, ql2, qi2);
         return;
     }
 #endif
-    fp_eval_ops<T, MATH, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast, th2, t2, qv2,
-                              ql2, qi2);
+    fp_eval_ops<T, MATH, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast, th2,
+                                      t2, qv2, ql2, qi2);
 }
 
-// Moist-adiabat fixed point for one sub-step from the cold start (:428-480).
-// Returns false when the iteration limit is exceeded (the reference then
-// zeroes CAPE/CIN and returns, :465-474).
+// Moist-adiabat fixed point for one sub-step from the cold start (:428-480),
+// as the reference writes it.  Returns false when the iteration limit is
+// exceeded (the reference then zeroes CAPE/CIN and returns, :465-474).
 template <typename T, int MATH, bool ICE>
-XC_HD __forceinline__ bool solve_substep(T p1, T p2, T pi2, T t1, T th1, T qv1, T ql1,
-                                              T qi1, T qt, T thlast, T &th2, T &t2, T &qv2,
-                                              T &ql2, T &qi2, LaneStats &st)
+XC_HD __forceinline__ bool solve_substep_ops(T p2, T pi2, T logp, T t1, T th1, T qv1, T ql1,
+                                             T qi1, T qt, T &th2, T &t2, T &qv2, T &ql2, T &qi2,
+                                             LaneStats &st)
 {
-    using F = Fn<T, MATH>;
-    const T logp = F::log(F::div(p2, p1));
+    T thlast = th1;
     int i = 0;
     while (true) {
         i = i + 1;
-        fp_eval<T, MATH, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast, th2, t2, qv2,
-                              ql2, qi2);
+        fp_eval_ops<T, MATH, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast, th2,
+                                          t2, qv2, ql2, qi2);
         st.iterations++;
         if (i > 100) return false;
         const T d = th2 - thlast;
@@ -257,6 +318,132 @@ XC_HD __forceinline__ bool solve_substep(T p1, T p2, T pi2, T t1, T th1, T qv1, 
             return true;
         }
     }
+}
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// The accurate mode's loop on the device, over fp_eval_raw.  `more`: not
+// converged after 100 evaluations (the 101st ends the column whatever it
+// gives, :464); `ok`: every evaluation was in the raw kernels' range, and in
+// the regime.
+//
+// FEW = false, for launches that fill the device: a lane that has converged
+// leaves the loop, and an ice adiabat's wave leaves out, in each evaluation,
+// the phase none of its lanes still iterating has (its lanes climb their
+// columns together: most evaluations are above 0 degC or below -40 degC on
+// every lane.  2^20 columns of 137 levels, pseudo-ice: 16.9 ms without, 12.2
+// with the regimes).
+//
+// FEW = true, for launches of a wave or so per SIMD, which wait for every
+// instruction: a lane that has converged keeps its iterate, so the evaluations
+// it goes on taking part in give its result again, and an iteration costs one
+// compare, one select and one branch beside the evaluation, with no execution
+// masks.  The regime is the caller's (REGIME), once for the whole sub-step.
+// (4096 columns of 40 levels, pseudo-liquid: 652 us with masks, 573 without;
+// 524 288 columns of 37 levels: 3.08 ms with, 3.40 without.)
+template <bool ICE, bool PSEUDO, bool FEW, int REGIME>
+__device__ __forceinline__ void solve_raw(float p2, float pi2, float logp, float t1, float th1,
+                                          float qv1, float ql1, float qi1, float qt, float &th2,
+                                          float &t2, float &qv2, float &ql2, float &qi2,
+                                          bool &more, bool &ok, LaneStats &st)
+{
+    // running maximum (minimum) by the median with an infinity the optimiser
+    // does not know (one instruction, no canonicalisation)
+    float inf = INFINITY;
+    __asm__("" : "+s"(inf));
+    float x = th1, worst = 0.0f, tlo = 1e30f, thi = 0.0f, arg;
+    int i = 0;
+    more = false;
+#define XC_EVAL(R)                                                                              \
+    fp_eval_raw<ICE, PSEUDO, R>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, x, th2, t2, qv2, ql2, \
+                                qi2, arg)
+    for (;;) {
+        if constexpr (ICE && !FEW) {
+            const float tx = x * pi2;
+            if (__builtin_amdgcn_ballot_w64(!regime_hot(p2, tx)) == 0) XC_EVAL(REG_LIQUID);
+            else if (__builtin_amdgcn_ballot_w64(!regime_cold(p2, tx)) == 0) XC_EVAL(REG_ICE);
+            else XC_EVAL(REG_MIXED);
+        } else {
+            XC_EVAL(REGIME);
+        }
+        worst = __builtin_amdgcn_fmed3f(worst, __builtin_fabsf(arg), inf);
+        if (REGIME != REG_MIXED) {
+            tlo = __builtin_amdgcn_fmed3f(tlo, t2, -inf);
+            thi = __builtin_amdgcn_fmed3f(thi, t2, inf);
+        }
+        const float d = th2 - x;
+        const bool go = __builtin_fabsf(d) > Phys<float>::converge;
+        st.iterations += !FEW || go ? 1 : 0;
+        if constexpr (FEW) {
+            x = go ? x + 0.3f * d : x;
+            if (__builtin_amdgcn_ballot_w64(go) == 0) break;
+        } else {
+            if (!go) break;
+            x = x + 0.3f * d;
+        }
+        // (the empty statement keeps this exit apart from the other one:
+        // joined, the two conditions cost a dozen scalar instructions per
+        // iteration)
+        if (++i == 100) {
+            more = go;
+            __asm__ volatile("");
+            break;
+        }
+    }
+#undef XC_EVAL
+    st.iterations += FEW || more ? 1 : 0;
+    // (a NaN does not enter `worst`, but `arg` keeps it: the lane's iterate
+    // no longer changes)
+    ok = worst < EXP_SMALL_MAX && arg_small(arg);
+    if (REGIME == REG_LIQUID) ok = ok && regime_hot(p2, tlo) && regime_hot(p2, thi);
+    if (REGIME == REG_ICE) ok = ok && regime_cold(p2, tlo) && regime_cold(p2, thi);
+}
+#endif
+
+// The same; on the device the accurate mode iterates with solve_raw.  With
+// few waves an ice adiabat's regime is chosen once per sub-step, from its
+// first iterate with a margin for the ones that follow (their temperatures
+// rise with the latent heat), and checked after the loop.  A sub-step that
+// left the raw kernels' range is solved again from its start with the
+// library's operations, whose iterates up to there are the same.
+template <typename T, int MATH, bool ICE, bool PSEUDO, bool FEW>
+XC_HD __forceinline__ bool solve_substep(T p1, T p2, T pi2, T t1, T th1, T qv1, T ql1, T qi1,
+                                         T qt, T &th2, T &t2, T &qv2, T &ql2, T &qi2,
+                                         LaneStats &st)
+{
+    const T logp = log_ratio<T, MATH>(p2, p1);
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (sizeof(T) == 4 && MATH == MATH_ACCURATE) {
+        bool more = false, ok = false;
+        const uint32_t it0 = st.iterations;
+        bool done = false;   // wave-uniform
+        if constexpr (ICE && FEW) {
+            const float tx = th1 * pi2;
+            if (__builtin_amdgcn_ballot_w64(!regime_hot(p2, tx - 0.1f)) == 0) {
+                solve_raw<ICE, PSEUDO, true, REG_LIQUID>(p2, pi2, logp, t1, th1, qv1, ql1, qi1,
+                                                         qt, th2, t2, qv2, ql2, qi2, more, ok,
+                                                         st);
+                done = __builtin_amdgcn_ballot_w64(!ok) == 0;
+            } else if (__builtin_amdgcn_ballot_w64(!regime_cold(p2, tx + 3.0f)) == 0) {
+                solve_raw<ICE, PSEUDO, true, REG_ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt,
+                                                      th2, t2, qv2, ql2, qi2, more, ok, st);
+                done = __builtin_amdgcn_ballot_w64(!ok) == 0;
+            }
+        }
+        if (!done) {
+            st.iterations = it0;
+            solve_raw<ICE, PSEUDO, FEW, REG_MIXED>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, th2,
+                                                   t2, qv2, ql2, qi2, more, ok, st);
+            if (__builtin_expect(!ok, 0)) {
+                st.iterations = it0;
+                return solve_substep_ops<T, MATH_LIB, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1,
+                                                           qt, th2, t2, qv2, ql2, qi2, st);
+            }
+        }
+        return !more;
+    }
+#endif
+    return solve_substep_ops<T, MATH, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, th2, t2,
+                                           qv2, ql2, qi2, st);
 }
 
 // Parcel source (:257-379): chooses the starting level kmax, the parcel's
@@ -571,9 +758,9 @@ struct NoLog {
 };
 
 // Reference driver: nested loops, cold start.  LEVELS: also the LFC and EL
-// (LevelTrack).
+// (LevelTrack).  FEW: solve_raw's loop for launches of few waves.
 template <typename T, int MATH, bool ICE, bool PSEUDO, class C, class LOG = NoLog,
-          bool LEVELS = false>
+          bool LEVELS = false, bool FEW = false>
 XC_HD void cape_column(const C &col, int nk, T pinc, int source, T ml_depth,
                        ColumnOut<T> &out, LaneStats &st, const LOG &log = LOG())
 {
@@ -613,8 +800,8 @@ XC_HD void cape_column(const C &col, int nk, T pinc, int source, T ml_depth,
             pi2 = Fn<T, MATH>::pow(p2 * K::rp00, K::rddcp);
             st.substeps++;
             const uint32_t it0 = st.iterations;
-            const bool ok = solve_substep<T, MATH, ICE>(p1, p2, pi2, t1, th1, qv1, ql1, qi1, qt,
-                                                        th1, th2, t2, qv2, ql2, qi2, st);
+            const bool ok = solve_substep<T, MATH, ICE, PSEUDO, FEW>(
+                p1, p2, pi2, t1, th1, qv1, ql1, qi1, qt, th2, t2, qv2, ql2, qi2, st);
             if (first_sub) st.first += st.iterations - it0;
             first_sub = false;
             if (!ok) {
@@ -856,7 +1043,7 @@ struct WarmAscent {
             qi1 = PSEUDO ? T(0.0) : qi2;
             p2 = p2 - dp;
             pi2 = F::pow(p2 * K::rp00, K::rddcp);
-            logp = F::log(F::div(p2, p1));
+            logp = log_ratio<T, MATH>(p2, p1);
             T g = th1;
             if (!predict) {
                 // every sub-step cold: the flattened loop without prediction
@@ -891,8 +1078,8 @@ struct WarmAscent {
             st.blocks |= 4u << rep;
             it = it + 1;
             const T x = thlast;
-            fp_eval<T, MATH, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, x, th2, t2, qv2,
-                                  ql2, qi2);
+            fp_eval<T, MATH, ICE, PSEUDO>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, x, th2, t2,
+                                          qv2, ql2, qi2);
             st.iterations++;
             if (first_sub) st.first++;
             const T d = th2 - x;

@@ -159,10 +159,27 @@ __device__ __forceinline__ int64_t out_col(const CapeGridArgs &a, int64_t col)
 // column per lane.  STATS: accumulate the work counters into a.stats (a
 // separate instantiation, so that the counters do not occupy registers in
 // the timed kernels).  LEVELS: also the LFC and EL (a.p_lfc, a.p_el).
-template <typename T, typename IDX, bool ICE, bool PSEUDO, bool STATS, bool LEVELS = false>
-__global__ void __launch_bounds__(256) cape_grid_kernel(CapeGridArgs a)
+// FEW (small launches, see few_columns): `cpw` columns to a wave, the lanes
+// beyond them on its columns again.  (Waves with few lanes switched on run
+// slowly: with fewer than about 12 the same instructions took up to three
+// times as many cycles, so 4096 columns at 4 to a wave took 1.6 ms with the
+// other lanes off and 0.57 ms with them repeating columns.)
+template <typename T, typename IDX, bool ICE, bool PSEUDO, bool STATS, bool LEVELS = false,
+          bool FEW = false>
+__global__ void __launch_bounds__(256) cape_grid_kernel(CapeGridArgs a, int cpw)
 {
-    const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t col;
+    bool own = true;   // this lane stores its column's outputs
+    if constexpr (FEW) {
+        const int lane = threadIdx.x & 63;
+        const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * cpw;
+        if (first >= a.ncol) return;
+        const int m = a.ncol - first < cpw ? (int)(a.ncol - first) : cpw;
+        col = first + lane % m;
+        own = lane < m;
+    } else {
+        col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    }
     SigmaCol<IDX> c{};
     int nk = 0;
     const bool in_grid = column_at(a, col, c, nk);
@@ -174,12 +191,13 @@ __global__ void __launch_bounds__(256) cape_grid_kernel(CapeGridArgs a)
         ColumnOut<T> o;
         if (c.ts > 0.0f) {
             ran = true;
-            cape_column<T, XC_MATH, ICE, PSEUDO, SigmaCol<IDX>, NoLog, LEVELS>(
+            cape_column<T, XC_MATH, ICE, PSEUDO, SigmaCol<IDX>, NoLog, LEVELS, FEW>(
                 c, nk, T(a.pinc), a.source, T(a.ml_depth), o, st);
         } else {
             o.cape = T(0); o.cin = T(0); o.zout = T(0); o.mulvl = 0;
             o.p_lfc = T(NAN); o.p_el = T(NAN);
         }
+        if (!own) return;
         cape[col] = o.cape;
         cin[col] = o.cin;
         a.mulvl[col] = o.mulvl;
@@ -559,18 +577,59 @@ hipError_t launch_srh(const CapeGridArgs &a, dim3 grid, int block, hipStream_t s
     return hipGetLastError();
 }
 
-template <typename T, typename IDX, bool STATS, bool LEVELS>
-hipError_t launch_cape_s(const CapeGridArgs &a, int block, hipStream_t s)
+// Columns per wave of a plain launch of at most two waves per SIMD, 0 for a
+// larger one.  The lanes of a wave iterate each sub-step until the slowest
+// has converged, and a SIMD with one wave takes as long for one column as for
+// 64, so a small grid is spread over the SIMDs: 1024 columns of 40 levels,
+// pseudo-liquid, take 477 us one to a wave and 574 us 64 to a wave; 65 536 of
+// 137 levels, pseudo-ice, 1.41 ms with the small launches' loop and 1.71
+// without; 131 072, 2.24 and 2.28; 262 144, 4.00 and 3.81.
+inline int few_columns(int64_t ncol)
 {
-    dim3 grid((unsigned)((a.ncol + block - 1) / block));
+    static const int simds = [] {
+        int dev = 0, ncu = 0;
+        (void)hipGetDevice(&dev);
+        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+        return 4 * (ncu > 0 ? ncu : 256);
+    }();
+    if (ncol > (int64_t)2 * 64 * simds) return 0;
+    const int64_t c = (ncol + simds - 1) / simds;
+    return c < 64 ? (int)c : 64;
+}
+
+template <typename T, typename IDX, bool STATS, bool LEVELS, bool FEW>
+hipError_t launch_cape_s(const CapeGridArgs &a, int block, int cpw, hipStream_t s)
+{
+    if (FEW) block = 256;
+    const int per = FEW ? 4 * cpw : block;
+    const dim3 grid((unsigned)((a.ncol + per - 1) / per));
     switch (a.adiabat) {
-    case 1: cape_grid_kernel<T, IDX, false, true, STATS, LEVELS><<<grid, block, 0, s>>>(a); break;
-    case 2: cape_grid_kernel<T, IDX, false, false, STATS, LEVELS><<<grid, block, 0, s>>>(a); break;
-    case 3: cape_grid_kernel<T, IDX, true, true, STATS, LEVELS><<<grid, block, 0, s>>>(a); break;
-    case 4: cape_grid_kernel<T, IDX, true, false, STATS, LEVELS><<<grid, block, 0, s>>>(a); break;
+    case 1:
+        cape_grid_kernel<T, IDX, false, true, STATS, LEVELS, FEW><<<grid, block, 0, s>>>(a, cpw);
+        break;
+    case 2:
+        cape_grid_kernel<T, IDX, false, false, STATS, LEVELS, FEW><<<grid, block, 0, s>>>(a, cpw);
+        break;
+    case 3:
+        cape_grid_kernel<T, IDX, true, true, STATS, LEVELS, FEW><<<grid, block, 0, s>>>(a, cpw);
+        break;
+    case 4:
+        cape_grid_kernel<T, IDX, true, false, STATS, LEVELS, FEW><<<grid, block, 0, s>>>(a, cpw);
+        break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+template <typename T, typename IDX, bool STATS, bool LEVELS>
+hipError_t launch_cape_f(const CapeGridArgs &a, int block, hipStream_t s)
+{
+    // the counted launches keep the large grids' loop
+    if constexpr (!STATS) {
+        if (const int cpw = few_columns(a.ncol))
+            return launch_cape_s<T, IDX, STATS, LEVELS, true>(a, block, cpw, s);
+    }
+    return launch_cape_s<T, IDX, STATS, LEVELS, false>(a, block, 0, s);
 }
 
 // 32-bit element offsets when every index of the profile arrays fits (the
@@ -580,13 +639,13 @@ template <typename T>
 hipError_t launch_cape(const CapeGridArgs &a, int block, hipStream_t s)
 {
     if (a.p_lfc && a.stats) return hipErrorInvalidValue;
-    if (a.stats) return launch_cape_s<T, uint64_t, true, false>(a, block, s);
+    if (a.stats) return launch_cape_f<T, uint64_t, true, false>(a, block, s);
     const bool fits = (uint64_t)a.ncol * (uint64_t)a.nk_in < ((uint64_t)1 << 32);
     if (a.p_lfc)
-        return fits ? launch_cape_s<T, uint32_t, false, true>(a, block, s)
-                    : launch_cape_s<T, uint64_t, false, true>(a, block, s);
-    return fits ? launch_cape_s<T, uint32_t, false, false>(a, block, s)
-                : launch_cape_s<T, uint64_t, false, false>(a, block, s);
+        return fits ? launch_cape_f<T, uint32_t, false, true>(a, block, s)
+                    : launch_cape_f<T, uint64_t, false, true>(a, block, s);
+    return fits ? launch_cape_f<T, uint32_t, false, false>(a, block, s)
+                : launch_cape_f<T, uint64_t, false, false>(a, block, s);
 }
 
 // Blocks of the persistent ascent: as many as the device holds at once, never

@@ -63,44 +63,40 @@ template <> struct Phys<double> {
 
 // ---- device kernels of the accurate mode -----------------------------------
 //
-// Division: the IEEE quotient from the hardware reciprocal and Markstein's
-// corrections -- y = 1/b refined by one Newton step, q = a y corrected twice
-// by the exact residual a - b q (fma).  These are the steps of the compiler's
-// own IEEE division without its operand scaling and special-value fix-up, so
-// where that scaling is the identity -- a, b and a/b normal, |b| < 2^126 --
-// the result is the same correctly rounded quotient, bit for bit.  A zero,
-// infinite or NaN operand gives NaN; subnormal or huge operands give a wrong
-// value.  Callers make sure of the range (the fixed-point evaluation below
-// re-evaluates with IEEE division whenever its result is not finite).
-__device__ __forceinline__ float div_raw(float a, float b)
+// Division: the correctly rounded quotient by Markstein's theorem: with y the
+// correctly rounded 1/b, q = RN(a y) and one correction by the exact residual
+// a - b q (fma) give RN(a/b).  The hardware reciprocal with one Newton step
+// is the correctly rounded one: compared on the device with IEEE 1/b over
+// every 23-bit mantissa at seven exponents from 2^-97 to 2^73, none differs
+// (the quotient has one correction fewer than the compiler's sequence, which
+// allows for an inexact reciprocal; 8.6e9 random quotients, none differs).
+// So for a, b and a/b normal, |b| < 2^126, the result is the IEEE quotient
+// bit for bit.  A zero, infinite or NaN operand (a zero dividend apart) gives
+// NaN; subnormal or huge operands give a wrong value.  Callers make sure of
+// the range (the fixed-point evaluation re-evaluates with IEEE division
+// whenever its result is not finite).
+__device__ __forceinline__ float rcp_rn(float b)
 {
     const float y0 = __builtin_amdgcn_rcpf(b);
     const float e = __builtin_fmaf(-b, y0, 1.0f);
-    const float y = __builtin_fmaf(e, y0, y0);
-    const float q0 = a * y;
-    const float r0 = __builtin_fmaf(-b, q0, a);
-    const float q1 = __builtin_fmaf(r0, y, q0);
-    const float r1 = __builtin_fmaf(-b, q1, a);
-    return __builtin_fmaf(r1, y, q1);
+    return __builtin_fmaf(e, y0, y0);
 }
 
-// Two quotients over one divisor, sharing the refined reciprocal (each
-// quotient's steps are div_raw's).
-__device__ __forceinline__ void div2_raw(float a1, float a2, float b, float &q1o, float &q2o)
+// a / b from y = rcp_rn(b)
+__device__ __forceinline__ float div_by(float a, float b, float y)
 {
-    const float y0 = __builtin_amdgcn_rcpf(b);
-    const float e = __builtin_fmaf(-b, y0, 1.0f);
-    const float y = __builtin_fmaf(e, y0, y0);
-    float q = a1 * y;
-    float r = __builtin_fmaf(-b, q, a1);
-    q = __builtin_fmaf(r, y, q);
-    r = __builtin_fmaf(-b, q, a1);
-    q1o = __builtin_fmaf(r, y, q);
-    q = a2 * y;
-    r = __builtin_fmaf(-b, q, a2);
-    q = __builtin_fmaf(r, y, q);
-    r = __builtin_fmaf(-b, q, a2);
-    q2o = __builtin_fmaf(r, y, q);
+    const float q = a * y;
+    const float r = __builtin_fmaf(-b, q, a);
+    return __builtin_fmaf(r, y, q);
+}
+
+__device__ __forceinline__ float div_raw(float a, float b) { return div_by(a, b, rcp_rn(b)); }
+
+// The smaller of two numbers, NaN if either is (one instruction; fmn below
+// for numbers).
+__device__ __forceinline__ float min_nan(float a, float b)
+{
+    return __builtin_elementwise_minimum(a, b);
 }
 
 // a / c for a divisor fixed per call, with rc = RN(1/c) computed once:
@@ -132,6 +128,37 @@ __device__ __forceinline__ float exp_core(float x)
     const float n = __builtin_rintf(ph);
     const float f = (ph - n) + pl;
     return __builtin_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+}
+
+// exp(x) for |x| < EXP_SMALL_MAX: exp_core's nearest integer is 0 there, so
+// its reduction and scaling drop out (exp_core's value bit for bit: compared
+// over every such float on the device).
+constexpr float EXP_SMALL_MAX = 0.34f;   // 0.34 log2(e) < 1/2
+
+__device__ __forceinline__ float exp_small(float x)
+{
+    constexpr float L2E = 0x1.715476p+0f;
+    constexpr float L2E_LO = 0x1.4ae0bep-26f;
+    const float ph = x * L2E;
+    float pl = __builtin_fmaf(x, L2E, -ph);
+    pl = __builtin_fmaf(x, L2E_LO, pl);
+    return __builtin_amdgcn_exp2f(ph + pl);
+}
+
+// ln x: the hardware log2 times ln 2 as a double-float (ln 2's bit patterns
+// 0x3f317217, 0x3377d1cf), the device library's steps without its scaling of
+// subnormals and its infinity select: the library's value for every float
+// from 1e-30 to 1e30 (compared over all of them on the device); -inf for 0,
+// NaN for a negative or NaN x.
+__device__ __forceinline__ float log_core(float x)
+{
+    constexpr float LN2 = 0x1.62e42ep-1f;
+    constexpr float LN2_LO = 0x1.efa39ep-25f;
+    const float l = __builtin_amdgcn_logf(x);
+    const float h = l * LN2;
+    float r = __builtin_fmaf(l, LN2, -h);
+    r = __builtin_fmaf(l, LN2_LO, r);
+    return h + r;
 }
 
 // x^y for 0 < x < 2^126, |y| <= 1 (the Exner function and theta-e's power):
