@@ -64,6 +64,31 @@ def test_loss_grad_matches_oracle(torch):
         assert err <= 1e-3 * scale + 1e-7, name
 
 
+@pytest.mark.parametrize('n', [1, 31, 64, 65, 200, 64 * 256, 64 * 256 + 1, 40_000])
+def test_loss_grad_tiles(torch, n):
+    """Batches of one tile of 64 samples, a partly filled one, one tile per
+    block and more.  A hidden value within FP32 error of a BF16 rounding
+    boundary may round the other way, which moves one sample's products by
+    2^-8 of themselves: that much of a block's largest entry for few samples,
+    the mean of many otherwise."""
+    from xcape_amd import surrogate
+    theta = _theta(4)
+    rng = np.random.default_rng(n)
+    x = rng.normal(0, 1, (n, 3)).astype(np.float32)
+    t = rng.normal(0, 1, n).astype(np.float32)
+    loss, g = surrogate.loss_grad(_t(torch, theta), _t(torch, x), _t(torch, t))
+    loss2, g2 = surrogate.loss_grad(_t(torch, theta), _t(torch, x), _t(torch, t))
+    assert torch.equal(g, g2) and torch.equal(loss, loss2)
+    g = g.cpu().numpy().astype(np.float64)
+    ref_loss, ref_g = mo.loss_and_grad(theta.astype(np.float64), x.astype(np.float64), t,
+                                       bf16_round=True)
+    tol = 2.0 ** -8 if n < 1000 else 1e-3
+    assert abs(loss.item() - ref_loss) <= tol * ref_loss
+    for name, (lo, hi) in BLOCKS.items():
+        scale = np.abs(ref_g[lo:hi]).max()
+        assert np.abs(g[lo:hi] - ref_g[lo:hi]).max() <= tol * scale + 1e-7, name
+
+
 def test_forward_matches_oracle(torch):
     from xcape_amd import _hip
     theta = _theta(2)

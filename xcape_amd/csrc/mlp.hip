@@ -3,13 +3,13 @@
 //
 // Training step (all FP32 accumulation; BF16 rounding where the inference
 // kernel rounds, so the trained network is the one the ascent evaluates):
-//   mlp_forward_store  one thread per sample: z1 = W1 u + b1, h1 = bf16(gelu(z1)),
-//                      z2 = W2 h1 + b2, h2 = gelu(z2), y = w3 . h2 + b3
-//   mlp_backward_rows  one thread per sample: dy = 2 (y - t) / n,
-//                      dz2 = dy w3 gelu'(z2), dz1 = (W2^T dz2) gelu'(z1)
-//   mlp_weight_grads   one block per hidden unit: sums over the batch of the
-//                      per-sample outer products (fixed order: deterministic)
-//   mlp_adam           Adam on the FP32 master vector
+//   mlp_train       64 samples at a time through the whole step in LDS --
+//                   z1 = W1 u + b1, h1 = bf16(gelu(z1)), z2 = W2 h1 + b2,
+//                   h2 = gelu(z2), y = w3 . h2 + b3, dy = 2 (y - t) / n,
+//                   dz2 = dy w3 gelu'(z2), dz1 = (W2^T dz2) gelu'(z1) -- and
+//                   the block's sums of the weight gradients
+//   mlp_grad_sum    the blocks' sums added up (fixed order: deterministic)
+//   mlp_adam        Adam on the FP32 master vector
 // The gradient is the straight-through one: the BF16 rounding is treated as
 // the identity in the backward pass.
 #include <hip/hip_runtime.h>
@@ -47,129 +47,252 @@ __device__ __forceinline__ void load_weights(const float *theta, FwdWeights &w)
     __syncthreads();
 }
 
-// forward for one sample; optionally stores z1, h1 (BF16-rounded), z2, h2
-__device__ __forceinline__ float forward_one(const FwdWeights &w, const float *u, float *z1s,
-                                             float *h1s, float *z2s, float *h2s)
+// forward for one sample
+__device__ __forceinline__ float forward_one(const FwdWeights &w, const float *u)
 {
     float h1[H];
 #pragma unroll
     for (int j = 0; j < H; ++j) {
         const float z = w.b1[j] + w.w1[3 * j] * u[0] + w.w1[3 * j + 1] * u[1] + w.w1[3 * j + 2] * u[2];
         h1[j] = bf16_round(gelu_f(z));
-        if (z1s) { z1s[j] = z; h1s[j] = h1[j]; }
     }
     float y = w.b3;
     for (int i = 0; i < H; ++i) {
         float z = w.b2[i];
 #pragma unroll
         for (int j = 0; j < H; ++j) z += w.w2[i * H + j] * h1[j];
-        const float h = gelu_f(z);
-        if (z2s) { z2s[i] = z; h2s[i] = h; }
-        y += w.w3[i] * h;
+        y += w.w3[i] * gelu_f(z);
     }
     return y;
 }
 
-__global__ void __launch_bounds__(256) mlp_forward_store(const float *x, int64_t n,
-                                                         const float *theta, float *y, float *Z1,
-                                                         float *H1, float *Z2, float *H2)
+__global__ void __launch_bounds__(256) mlp_forward(const float *x, int64_t n, const float *theta,
+                                                   float *y)
 {
     __shared__ FwdWeights w;
     load_weights(theta, w);
     const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
     const float u[3] = {x[3 * s], x[3 * s + 1], x[3 * s + 2]};
-    if (Z1)
-        y[s] = forward_one(w, u, Z1 + s * H, H1 + s * H, Z2 + s * H, H2 + s * H);
-    else
-        y[s] = forward_one(w, u, nullptr, nullptr, nullptr, nullptr);
+    y[s] = forward_one(w, u);
 }
 
-__global__ void __launch_bounds__(256) mlp_backward_rows(const float *y, const float *t,
-                                                         int64_t n, const float *theta,
-                                                         const float *Z1, const float *Z2,
-                                                         float *dZ1, float *dZ2, float *dy)
+// ---- the training step's gradients ------------------------------------------
+//
+// A block takes tiles of 64 samples in turn and keeps everything of a tile in
+// LDS and registers; with one pass per layer over global memory instead, the
+// activations and their gradients (6 arrays of 64 floats per sample) went
+// through HBM between three launches, and the weight gradients' sums ran on 65
+// blocks.  A step at 16 384 samples (gradients and Adam) took 334 us so and
+// takes 43 us here; what is left is its three launches.
+//
+// The products over 64 units or 64 samples run on the matrix cores: the
+// forward's W2 h1 in BF16 (both operands are BF16 values: exact products, FP32
+// sums), the backward's W2^T dz2 and dz2 h1^T in FP32, since dz2 is FP32.
+// Wave (tm, tn) = (wave / 2, wave % 2) owns one 32 x 32 tile of each product,
+// in the layout of v_mfma_f32_32x32x*: register r of lane (half, col) is
+// element [32 tm + 8 (r / 4) + 4 half + r % 4][32 tn + col].  Layer 1 is
+// computed in that layout too ([sample][unit]), so its slopes stay in the
+// registers where the backward product delivers dz1.
+constexpr int TT = 64;                 // samples per tile
+constexpr int TP = 65;                 // row pitch of the FP32 tiles in LDS (distinct banks)
+constexpr int TPB = 36;                // row pitch of the BF16 tiles, words (16-byte rows)
+constexpr int GRAD_ROW = MLP_NPARAMS + 1;   // a block's sums: the gradient, then the loss
+constexpr int TRAIN_BLOCKS = 256;      // one per CU (the tiles take 88 KB of its LDS)
+
+struct TrainLds {
+    float w2[H * H];                   // BF16-rounded, [i][j]
+    float h1[TT * TP];                 // [sample][j]
+    float dz2[H * TP];                 // [i][sample]
+    float h2[H * TP];                  // [i][sample]
+    uint32_t w2b[H * TPB];             // BF16 pairs, [i][j]
+    uint32_t h1b[TT * TPB];            // BF16 pairs, [sample][j]
+    float x[TT * 3], t[TT], y[2][TT], dy[TT];
+    float b2[H], w3[H], red[4][H];
+};
+
+// gelu_f and gelu_grad_f of one argument
+__device__ __forceinline__ void gelu_both(float z, float &h, float &slope)
 {
-    __shared__ FwdWeights w;
-    load_weights(theta, w);
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const float g = 2.0f * (y[s] - t[s]) / (float)n;
-    dy[s] = g;
-    float dz2[H];
-#pragma unroll
-    for (int i = 0; i < H; ++i) {
-        dz2[i] = g * w.w3[i] * gelu_grad_f(Z2[s * H + i]);
-        dZ2[s * H + i] = dz2[i];
-    }
-    for (int j = 0; j < H; ++j) {
-        float d = 0.0f;
-#pragma unroll
-        for (int i = 0; i < H; ++i) d += w.w2[i * H + j] * dz2[i];
-        dZ1[s * H + j] = d * gelu_grad_f(Z1[s * H + j]);
-    }
+    const float c = 0.7978845608028654f, a = 0.044715f;
+    const float u = c * (z + a * z * z * z);
+    const float e = __expf(2.0f * u);
+    const float t = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
+    h = 0.5f * z * (1.0f + t);
+    slope = 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * c * (1.0f + 3.0f * a * z * z);
 }
 
-// Block b < 64: gradients owned by hidden unit b (row b of W2, W1, entries b
-// of b1, b2, w3).  Block 64: b3 and the loss.  Each thread sums a strided
-// subset of the samples; the block then reduces in a fixed tree.
-constexpr int WG_THREADS = 128;
-
-__global__ void __launch_bounds__(WG_THREADS) mlp_weight_grads(const float *x, const float *t,
-                                                        const float *y, int64_t n,
-                                                        const float *H1, const float *H2,
-                                                        const float *dZ1, const float *dZ2,
-                                                        const float *dy, float *grad,
-                                                        float *loss)
+// grid: at most TRAIN_BLOCKS blocks, block b takes tiles b, b + grid, ...;
+// part: GRAD_ROW floats per block
+__global__ void __launch_bounds__(256) mlp_train(const float *x, const float *t, int64_t n,
+                                                 const float *theta, float *part)
 {
-    constexpr int NV = H + 3 + 3;   // dW2 row (64), dW1 row (3), db1, db2, dw3
-    __shared__ float red[NV][WG_THREADS];
-    const int b = blockIdx.x;
-    float acc[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) acc[v] = 0.0f;
-    if (b < H) {
-        for (int64_t s = threadIdx.x; s < n; s += blockDim.x) {
-            const float d2 = dZ2[s * H + b], d1 = dZ1[s * H + b];
-#pragma unroll
-            for (int j = 0; j < H; ++j) acc[j] += d2 * H1[s * H + j];
-            acc[H + 0] += d1 * x[3 * s];
-            acc[H + 1] += d1 * x[3 * s + 1];
-            acc[H + 2] += d1 * x[3 * s + 2];
-            acc[H + 3] += d1;
-            acc[H + 4] += d2;
-            acc[H + 5] += dy[s] * H2[s * H + b];
-        }
-    } else {
-        for (int64_t s = threadIdx.x; s < n; s += blockDim.x) {
-            acc[0] += dy[s];
-            const float r = y[s] - t[s];
-            acc[1] += r * r;
-        }
+    __shared__ TrainLds L;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int half = lane >> 5, col = lane & 31, tm = wave >> 1, tn = wave & 1;
+    const int row0 = 32 * tm + 4 * half;           // row of register r: row0 + 8 (r / 4) + r % 4
+    const int j = 32 * tn + col;
+    for (int i = tid; i < H * H; i += 256) {
+        const uint16_t b = bf16_bits(theta[MLP_OFF_W2 + i]);
+        L.w2[i] = __uint_as_float((uint32_t)b << 16);
+        reinterpret_cast<uint16_t *>(L.w2b)[(i / H) * 2 * TPB + i % H] = b;
     }
+    if (tid < H) {
+        L.b2[tid] = theta[MLP_OFF_B2 + tid];
+        L.w3[tid] = bf16_round(theta[MLP_OFF_W3 + tid]);
+    }
+    const float b3 = theta[MLP_OFF_B3];
+    const float b1 = theta[MLP_OFF_B1 + j];
+    const float w10 = bf16_round(theta[MLP_OFF_W1 + 3 * j]),
+                w11 = bf16_round(theta[MLP_OFF_W1 + 3 * j + 1]),
+                w12 = bf16_round(theta[MLP_OFF_W1 + 3 * j + 2]);
+    xc_f32x16 gw2 = {};
+    float gw10 = 0.0f, gw11 = 0.0f, gw12 = 0.0f, gb1 = 0.0f;   // unit j, this lane's samples
+    float gvec = 0.0f;            // threads 0 .. 63: dw3[tid]; 64 .. 127: db2[tid - 64]
+    float gb3 = 0.0f, loss = 0.0f;                             // threads 0 .. 63
+    const int64_t tiles = (n + TT - 1) / TT;
+    for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int64_t s0 = tile * TT;
+        const int ns = n - s0 < TT ? (int)(n - s0) : TT;
+        // samples past n: zero inputs, and dy = 0 below
+        if (tid < 3 * TT) L.x[tid] = tid < 3 * ns ? x[3 * s0 + tid] : 0.0f;
+        else if (tid - 3 * TT < TT) L.t[tid - 3 * TT] = tid - 3 * TT < ns ? t[s0 + tid - 3 * TT] : 0.0f;
+        __syncthreads();
+        // layer 1: samples row0 + .., unit j
+        float slope1[16];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) red[v][threadIdx.x] = acc[v];
-    __syncthreads();
-    for (int stride = WG_THREADS / 2; stride > 0; stride >>= 1) {
-        if ((int)threadIdx.x < stride) {
-#pragma unroll
-            for (int v = 0; v < NV; ++v) red[v][threadIdx.x] += red[v][threadIdx.x + stride];
+        for (int r = 0; r < 16; ++r) {
+            const int s = row0 + 8 * (r >> 2) + (r & 3);
+            const float z = b1 + w10 * L.x[3 * s] + w11 * L.x[3 * s + 1] + w12 * L.x[3 * s + 2];
+            float h;
+            gelu_both(z, h, slope1[r]);
+            const uint16_t b = bf16_bits(h);
+            L.h1[s * TP + j] = __uint_as_float((uint32_t)b << 16);
+            reinterpret_cast<uint16_t *>(L.h1b)[s * 2 * TPB + j] = b;
         }
         __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        if (b < H) {
-            for (int j = 0; j < H; ++j) grad[MLP_OFF_W2 + b * H + j] = red[j][0];
-            grad[MLP_OFF_W1 + 3 * b + 0] = red[H + 0][0];
-            grad[MLP_OFF_W1 + 3 * b + 1] = red[H + 1][0];
-            grad[MLP_OFF_W1 + 3 * b + 2] = red[H + 2][0];
-            grad[MLP_OFF_B1 + b] = red[H + 3][0];
-            grad[MLP_OFF_B2 + b] = red[H + 4][0];
-            grad[MLP_OFF_W3 + b] = red[H + 5][0];
-        } else {
-            grad[MLP_OFF_B3] = red[0][0];
-            if (loss) *loss = red[1][0] / (float)n;
+        // layer 2: units row0 + .., sample j; layer 3's partial sums
+        xc_f32x16 z2 = {};
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            const int k0 = 8 * kb + 4 * half;      // words
+            xc_bf16x8 a, b;
+            __builtin_memcpy(&a, &L.w2b[(32 * tm + col) * TPB + k0], 16);
+            __builtin_memcpy(&b, &L.h1b[j * TPB + k0], 16);
+            z2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, z2, 0, 0, 0);
         }
+        float slope2[16], part3 = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int i = row0 + 8 * (r >> 2) + (r & 3);
+            float h;
+            gelu_both(z2[r] + L.b2[i], h, slope2[r]);
+            L.h2[i * TP + j] = h;
+            part3 += L.w3[i] * h;
+        }
+        part3 += __shfl_xor(part3, 32, 64);
+        if (half == 0) L.y[tm][j] = part3;
+        __syncthreads();
+        if (tid < TT) {
+            const float r = tid < ns ? (b3 + L.y[0][tid] + L.y[1][tid]) - L.t[tid] : 0.0f;
+            const float g = 2.0f * r / (float)n;
+            L.dy[tid] = g;
+            gb3 += g;
+            loss += r * r;
+        }
+        __syncthreads();
+        const float dyj = L.dy[j];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int i = row0 + 8 * (r >> 2) + (r & 3);
+            L.dz2[i * TP + j] = dyj * L.w3[i] * slope2[r];
+        }
+        __syncthreads();
+        // dz1^T W2 (samples x units) and dz2 h1 (units x units)
+        xc_f32x16 d1 = {};
+#pragma unroll 8
+        for (int kk = 0; kk < 32; ++kk) {
+            const int k = 2 * kk + half;
+            d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(L.dz2[k * TP + 32 * tm + col],
+                                                      L.w2[k * H + j], d1, 0, 0, 0);
+            gw2 = __builtin_amdgcn_mfma_f32_32x32x2f32(L.dz2[(32 * tm + col) * TP + k],
+                                                       L.h1[k * TP + j], gw2, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int s = row0 + 8 * (r >> 2) + (r & 3);
+            const float d = d1[r] * slope1[r];
+            gw10 += d * L.x[3 * s];
+            gw11 += d * L.x[3 * s + 1];
+            gw12 += d * L.x[3 * s + 2];
+            gb1 += d;
+        }
+        if (tid < 2 * H) {
+            const float *v = tid < H ? L.h2 + tid * TP : L.dz2 + (tid - H) * TP;
+#pragma unroll 8
+            for (int s = 0; s < TT; ++s) gvec += tid < H ? L.dy[s] * v[s] : v[s];
+        }
+        __syncthreads();   // the tile's arrays are rewritten by the next one
+    }
+    // the block's sums
+    float *p = part + (size_t)blockIdx.x * GRAD_ROW;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        p[MLP_OFF_W2 + (row0 + 8 * (r >> 2) + (r & 3)) * H + j] = gw2[r];
+    if (tid < H) p[MLP_OFF_W3 + tid] = gvec;
+    else if (tid < 2 * H) p[MLP_OFF_B2 + tid - H] = gvec;
+    // unit j's sums: this lane's, its other half's, the other row tile's
+    gw10 += __shfl_xor(gw10, 32, 64);
+    gw11 += __shfl_xor(gw11, 32, 64);
+    gw12 += __shfl_xor(gw12, 32, 64);
+    gb1 += __shfl_xor(gb1, 32, 64);
+    if (tm == 1 && half == 0) {
+        L.red[0][j] = gw10;
+        L.red[1][j] = gw11;
+        L.red[2][j] = gw12;
+        L.red[3][j] = gb1;
+    }
+    __syncthreads();
+    if (tm == 0 && half == 0) {
+        p[MLP_OFF_W1 + 3 * j] = gw10 + L.red[0][j];
+        p[MLP_OFF_W1 + 3 * j + 1] = gw11 + L.red[1][j];
+        p[MLP_OFF_W1 + 3 * j + 2] = gw12 + L.red[2][j];
+        p[MLP_OFF_B1 + j] = gb1 + L.red[3][j];
+    }
+    if (wave == 0) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            gb3 += __shfl_xor(gb3, off, 64);
+            loss += __shfl_xor(loss, off, 64);
+        }
+        if (lane == 0) {
+            p[MLP_OFF_B3] = gb3;
+            p[MLP_NPARAMS] = loss;
+        }
+    }
+}
+
+// The blocks' sums of one parameter per lane: 16 rows of 64 lanes take every
+// 16th block's, and are added in order.
+__global__ void __launch_bounds__(1024) mlp_grad_sum(const float *part, int nblk, int64_t n,
+                                                     float *grad, float *loss)
+{
+    __shared__ float red[16][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int c = blockIdx.x * 64 + lane;
+    float v = 0.0f;
+    if (c < GRAD_ROW) {
+#pragma unroll 4
+        for (int b = w; b < nblk; b += 16) v += part[(size_t)b * GRAD_ROW + c];
+    }
+    red[w][lane] = v;
+    __syncthreads();
+    if (w == 0 && c < GRAD_ROW) {
+        v = red[0][lane];
+#pragma unroll
+        for (int k = 1; k < 16; ++k) v += red[k][lane];
+        if (c < MLP_NPARAMS) grad[c] = v;
+        else if (loss) *loss = v / (float)n;
     }
 }
 
@@ -262,7 +385,7 @@ int xcape_mlp_forward(const float *x, int64_t n, const float *theta, float *y, v
     if (!x || !theta || !y) return fail(XCAPE_EINVAL, "NULL argument");
     hipStream_t s = (hipStream_t)stream;
     const unsigned blocks = (unsigned)((n + 255) / 256);
-    mlp_forward_store<<<blocks, 256, 0, s>>>(x, n, theta, y, nullptr, nullptr, nullptr, nullptr);
+    mlp_forward<<<blocks, 256, 0, s>>>(x, n, theta, y);
     hipError_t e = hipGetLastError();
     return e ? hip_fail(e, "mlp_forward") : XCAPE_OK;
 }
@@ -274,19 +397,13 @@ int xcape_mlp_loss_grad(const float *x, const float *t, int64_t n, const float *
     if (rc || (rc = ensure_device())) return rc;
     if (!x || !t || !theta || !grad) return fail(XCAPE_EINVAL, "NULL argument");
     hipStream_t s = (hipStream_t)stream;
-    const size_t nh = (size_t)n * H;
-    DevBuf<float> y, Z1, H1, Z2, H2, dZ1, dZ2, dy;
+    const int64_t tiles = (n + TT - 1) / TT;
+    const int blocks = tiles < TRAIN_BLOCKS ? (int)tiles : TRAIN_BLOCKS;
+    DevBuf<float> part;
     hipError_t e;
-    if ((e = y.alloc(n, s)) || (e = Z1.alloc(nh, s)) || (e = H1.alloc(nh, s)) ||
-        (e = Z2.alloc(nh, s)) || (e = H2.alloc(nh, s)) || (e = dZ1.alloc(nh, s)) ||
-        (e = dZ2.alloc(nh, s)) || (e = dy.alloc(n, s)))
-        return hip_fail(e, "mlp workspace");
-    const unsigned blocks = (unsigned)((n + 255) / 256);
-    mlp_forward_store<<<blocks, 256, 0, s>>>(x, n, theta, y.ptr, Z1.ptr, H1.ptr, Z2.ptr, H2.ptr);
-    mlp_backward_rows<<<blocks, 256, 0, s>>>(y.ptr, t, n, theta, Z1.ptr, Z2.ptr, dZ1.ptr,
-                                             dZ2.ptr, dy.ptr);
-    mlp_weight_grads<<<H + 1, WG_THREADS, 0, s>>>(x, t, y.ptr, n, H1.ptr, H2.ptr, dZ1.ptr, dZ2.ptr,
-                                           dy.ptr, grad, loss);
+    if ((e = part.alloc((size_t)blocks * GRAD_ROW, s))) return hip_fail(e, "mlp workspace");
+    mlp_train<<<blocks, 256, 0, s>>>(x, t, n, theta, part.ptr);
+    mlp_grad_sum<<<(GRAD_ROW + 63) / 64, 1024, 0, s>>>(part.ptr, blocks, n, grad, loss);
     e = hipGetLastError();
     return e ? hip_fail(e, "mlp_loss_grad") : XCAPE_OK;
 }
