@@ -219,3 +219,45 @@ def test_fused_c4_shape_against_oracle(hip, oracle_lib):
     o = oracle_lib.cape(a[0], a[1], a[2], a[5], a[6], a[7], pinc=500., source=2, adiabat=3)
     assert np.all(cape_ok(f[0], o[0])) and np.all(cape_ok(f[1], o[1]))
     _cmp_srh(f[4:], oracle_lib.srh(*a, 3000.), 'fused C4')
+
+
+@pytest.mark.parametrize('p_shared', [False, True])
+@pytest.mark.parametrize('ncol,nk', [(1, 5), (63, 16), (64, 8), (65, 31), (129, 1), (700, 137),
+                                     (1003, 33)])
+def test_profiles_where_they_lie_match_level_major(hip, ncol, nk, p_shared):
+    """Column-contiguous profiles go to the kernel that computes a block of
+    columns' heights level by level, level-major ones to the lane per column:
+    the same arithmetic, the same bits, in every precision and input type, at
+    the edges of the blocks (64 columns) and of the windows (8 levels), with
+    heights that fall, NaN and values outside the fast kernels' range."""
+    import torch
+    if p_shared:
+        c = synthetic.pressure_columns(ncol, ncol, levels=np.linspace(1000, 100, max(nk, 2)),
+                                       winds=True)
+        nk = max(nk, 2)
+    else:
+        c = synthetic.sigma_columns(ncol, nk, ncol, winds=True)
+    if ncol > 500:
+        c['t'][5, 3] = np.nan
+        c['td'][7, nk // 2:] = np.nan
+        c['t'][9, nk - 3] = -300.0
+        c['td'][11] = -273.15
+        c['td'][15, nk - 2] = 1000.0
+        c['u'][13, 4] = np.nan
+        c['ps'][16] = 0.0
+        c['tds'][18] = -273.15
+        if not p_shared:
+            c['p'][3] = c['p'][3][::-1]
+            c['p'][8, 20] = c['p'][8, 19]
+            c['p'][10, nk - 1] = 0.0
+            c['p'][21, 25] = np.inf
+            c['p'][12] = -c['p'][12]
+    names = ('p', 't', 'td', 'u', 'v', 'ps', 'ts', 'tds', 'us', 'vs')
+    for dt in (np.float32, np.float64):
+        a = [torch.from_numpy(c[k].astype(dt)).cuda() for k in names]
+        b = [x.t().contiguous() if x.ndim == 2 else x for x in a]
+        for fp64 in (False, True):
+            for depth in (3000.0, 9000.0, 1.0):
+                kw = dict(depth=depth, fp64=fp64, inputs_f64=dt == np.float64, p_shared=p_shared)
+                for x, y in zip(hip.srh(*a, **kw), hip.srh(*b, level_major=True, **kw)):
+                    assert torch.equal(x.nan_to_num(nan=-7e7), y.nan_to_num(nan=-7e7))

@@ -1,7 +1,7 @@
 // Rectangular-grid kernels (sigma or shared pressure levels), included by
 // one translation unit per math mode with XC_MATH defined.
 //
-// Every kernel here reads level-major profiles, level k of column j at
+// The CAPE kernels read level-major profiles, level k of column j at
 // k * ls + j (the C-ABI stages column-contiguous input through the LDS
 // transpose first), so that the 64 lanes of a wave read 64 consecutive words
 // per level; one column per lane.  The plain method is one launch
@@ -154,6 +154,32 @@ __device__ __forceinline__ int64_t out_col(const CapeGridArgs &a, int64_t col)
 {
     return a.out_index ? (int64_t)a.out_index[col] : col;
 }
+
+template <typename TB>
+__device__ __forceinline__ void store_srh(const CapeGridArgs &a, int64_t col,
+                                          const SrhOutT<TB> &so)
+{
+    a.srh_rm[col] = so.srh_rm;
+    a.srh_lm[col] = so.srh_lm;
+    if (a.rm) {
+        TB *rm = static_cast<TB *>(a.rm), *lm = static_cast<TB *>(a.lm),
+           *mw = static_cast<TB *>(a.mean6);
+        rm[2 * col] = so.rm_u;
+        rm[2 * col + 1] = so.rm_v;
+        lm[2 * col] = so.lm_u;
+        lm[2 * col + 1] = so.lm_v;
+        mw[2 * col] = so.mean_u;
+        mw[2 * col + 1] = so.mean_v;
+    }
+}
+
+}  // namespace XC_NS
+}  // namespace xcape
+
+#include "srh_slab.h"
+
+namespace xcape {
+namespace XC_NS {
 
 // CAPE/CIN with the reference's loops and cold start (cape_column), one
 // column per lane.  STATS: accumulate the work counters into a.stats (a
@@ -531,7 +557,8 @@ __global__ void warm_reset_kernel(unsigned int *work, uint32_t ncol, uint32_t gr
     if (threadIdx.x < parts) work[threadIdx.x] = work_part_begin(ncol, threadIdx.x, parts);
 }
 
-// Storm-relative helicity chain, one column per lane.  TB: the storm-motion
+// Storm-relative helicity chain over level-major profiles, one column per lane
+// (column-contiguous ones: srh_slab_kernel).  TB: the storm-motion
 // precision (float: the reference's; double: the FP64 re-run).  TI: the
 // input element type (double: float64 profiles, which feed the FP64 heights
 // and helicity unrounded as the reference's f2py wrappers pass them).
@@ -553,23 +580,20 @@ srh_grid_kernel(CapeGridArgs a)
     c.vs = in_arr<TI>(a.vs)[col];
     SrhOutT<TB> so;
     srh_column<TB>(c, nk, a.depth, 2.0, so);
-    a.srh_rm[col] = so.srh_rm;
-    a.srh_lm[col] = so.srh_lm;
-    if (a.rm) {
-        TB *rm = static_cast<TB *>(a.rm), *lm = static_cast<TB *>(a.lm),
-           *mw = static_cast<TB *>(a.mean6);
-        rm[2 * col] = so.rm_u;
-        rm[2 * col + 1] = so.rm_v;
-        lm[2 * col] = so.lm_u;
-        lm[2 * col + 1] = so.lm_v;
-        mw[2 * col] = so.mean_u;
-        mw[2 * col + 1] = so.mean_v;
-    }
+    store_srh(a, col, so);
 }
 
 template <typename TB>
 hipError_t launch_srh(const CapeGridArgs &a, dim3 grid, int block, hipStream_t s)
 {
+    if (a.ls == 1) {   // column-contiguous profiles
+        const dim3 slabs((unsigned)((a.ncol + SRH_COLS - 1) / SRH_COLS));
+        if (a.in_f64)
+            srh_slab_kernel<TB, double><<<slabs, 256, 0, s>>>(a);
+        else
+            srh_slab_kernel<TB, float><<<slabs, 256, 0, s>>>(a);
+        return hipGetLastError();
+    }
     if (a.in_f64)
         srh_grid_kernel<TB, double><<<grid, block, 0, s>>>(a);
     else

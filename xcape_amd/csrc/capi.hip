@@ -193,74 +193,51 @@ int cape_block()
     return 256;
 }
 
-// Profile copies only the helicity launch reads (the winds of a combined
-// call), made on whichever stream runs that launch.
-struct HelicityStage {
-    const float *src[2];
-    float *dst[2];
-    int narr;
-    int64_t n, nk;
-};
-
-// The grid kernels read level-major profiles: with a column per lane, 64
+// The CAPE kernels read level-major profiles: with a column per lane, 64
 // lanes reading 64 different columns of column-contiguous arrays fetch 64
 // cache lines per level each, and on large grids the L2 cannot hold them
 // for the ~32 levels each line serves (measured on 2048x1024x137: 142 GB
 // fetched per ascent launch for 3.4 GB of profiles).  Level-major profiles go
 // straight to the kernels; column-contiguous ones are staged level-major
-// first through the LDS-tiled transpose.  run_grid works in chunks of
-// columns whose scratch fits in about 16 GiB: per chunk, one transpose launch
-// for the profile arrays the CAPE launches read (shared with the helicity
-// launch; none for level-major input), the warm-started ascent's scratch
-// (level environments and parcels), then the launches.  A combined call
-// copies the winds on the helicity's stream, where they run beside the CAPE
-// launches (beside the warm-started ascent, after its setup pass) instead of
-// ahead of them.
-hipError_t launch_grid(const CapeGridArgs &a, bool cape, bool srh, int math, hipStream_t s,
-                       const HelicityStage *hs = nullptr)
+// first through the LDS-tiled transpose.  The helicity chain reads either
+// layout where it lies.  run_grid works in chunks of columns whose scratch
+// fits in about 16 GiB: per chunk, one transpose launch for the profile arrays
+// the CAPE launches read (none for level-major input), the warm-started
+// ascent's scratch (level environments and parcels), then the launches.
+//
+// a: the CAPE launches' arguments; h: the helicity launch's (the same call
+// with the profiles as the caller laid them out).
+hipError_t launch_grid(const CapeGridArgs &a, const CapeGridArgs &h, bool cape, bool srh, int math,
+                       hipStream_t s)
 {
     hipError_t e = hipSuccess;
     if (cape && srh) {
-        // the helicity chain (memory- and FP64-bound) beside the ascent
-        // (FP32-bound): forked onto the thread's second stream after the
-        // work already queued on s, joined back before anything later on s
+        // the helicity chain (FP64-bound) beside the ascent (FP32-bound):
+        // forked onto the thread's second stream after the work already queued
+        // on s (after the setup pass of a warm start), joined back before
+        // anything later on s
         hipStream_t s2 = aux_stream();
         const hipEvent_t fork = thread_event(EV_FORK), join = thread_event(EV_JOIN),
                          setup = thread_event(EV_SETUP);
-        if (s2 && s2 != s && fork && join && hs && setup && a.warm != 0 && math != 2) {
-            // warm start with the winds to copy: the second stream starts after
-            // the setup pass, so that the copies run beside the ascent (bound by
-            // VALU issue) rather than beside the setup pass (which moves about
-            // as many bytes per microsecond as they do)
-            CapeGridArgs ac = a;
-            ac.setup_done = setup;
-            if ((e = launch_grid(ac, true, false, math, s)) != hipSuccess) return e;
-            if ((e = hipStreamWaitEvent(s2, setup, 0)) != hipSuccess) return e;
-            e = launch_transpose_levels(hs->src, hs->dst, hs->narr, hs->n, hs->nk, s2);
-            if (e == hipSuccess) e = launch_cape_grid_accurate(a, false, GRID_SRH, 256, s2);
-            const hipError_t er = hipEventRecord(join, s2);
-            if (e == hipSuccess) e = er;
-            // join even when a launch failed: s must not run ahead of s2
-            const hipError_t ej = hipStreamWaitEvent(s, join, 0);
-            return e != hipSuccess ? e : ej;
-        }
-        if (s2 && s2 != s && fork && join) {
-            if ((e = hipEventRecord(fork, s)) != hipSuccess ||
-                (e = hipStreamWaitEvent(s2, fork, 0)) != hipSuccess)
+        if (s2 && s2 != s && fork && join && setup) {
+            const bool warm = a.warm != 0 && math != 2;
+            if (warm) {
+                CapeGridArgs ac = a;
+                ac.setup_done = setup;
+                if ((e = launch_grid(ac, h, true, false, math, s)) != hipSuccess) return e;
+            } else if ((e = hipEventRecord(fork, s)) != hipSuccess) {
                 return e;
-            if (hs) e = launch_transpose_levels(hs->src, hs->dst, hs->narr, hs->n, hs->nk, s2);
-            if (e == hipSuccess) e = launch_cape_grid_accurate(a, false, GRID_SRH, 256, s2);
+            }
+            if ((e = hipStreamWaitEvent(s2, warm ? setup : fork, 0)) != hipSuccess) return e;
+            e = launch_cape_grid_accurate(h, false, GRID_SRH, 256, s2);
             const hipError_t er = hipEventRecord(join, s2);
             if (e == hipSuccess) e = er;
-            if (e == hipSuccess) e = launch_grid(a, true, false, math, s);
+            if (!warm && e == hipSuccess) e = launch_grid(a, h, true, false, math, s);
             // join even when a launch failed: s must not run ahead of s2
             const hipError_t ej = hipStreamWaitEvent(s, join, 0);
             return e != hipSuccess ? e : ej;
         }
     }
-    if (hs && (e = launch_transpose_levels(hs->src, hs->dst, hs->narr, hs->n, hs->nk, s)) !=
-                  hipSuccess)
-        return e;
     if (cape) {
         const int block = cape_block();
         if (math == 2)
@@ -273,34 +250,19 @@ hipError_t launch_grid(const CapeGridArgs &a, bool cape, bool srh, int math, hip
     }
     // the helicity chain keeps the reference's precisions in every math mode
     // but the FP64 one (storm motion in double)
-    if (srh) e = launch_cape_grid_accurate(a, math == 2, GRID_SRH, 256, s);
+    if (srh) e = launch_cape_grid_accurate(h, math == 2, GRID_SRH, 256, s);
     return e;
 }
 
 // Scratch floats per column of one run_grid chunk (staged profiles plus the
 // warm-started ascent's records); 0 when the call needs none.
-int64_t grid_scratch_floats(const CapeGridArgs &a0, bool cape, bool srh, int math)
+int64_t grid_scratch_floats(const CapeGridArgs &a0, bool cape, int math)
 {
-    const bool stage = a0.ls == 1 && a0.nk_in > 1 && !a0.in_f64;
+    const bool stage = cape && a0.ls == 1 && a0.nk_in > 1;
     const bool warm = cape && a0.warm != 0 && math != 2;
-    const int narr = stage ? 2 + (a0.p != nullptr) + (srh ? 2 : 0) : 0;
+    const int narr = stage ? 2 + (a0.p != nullptr) : 0;
     return (int64_t)narr * a0.nk_in +
            (warm ? warm_scratch_floats(a0.nk_in, a0.p_lfc != nullptr) : 0);
-}
-
-// A helicity-only call on at least this many column-contiguous columns
-// (XCAPE_SRH_PIPE_COLUMNS overrides it, read on every call; for tests) is
-// staged and computed in SRH_PARTS parts: each part's helicity launch runs on
-// the thread's second stream while the next part's profiles are copied.
-constexpr int SRH_PARTS = 4;
-
-int64_t srh_pipe_min_columns()
-{
-    if (const char *env = getenv("XCAPE_SRH_PIPE_COLUMNS")) {
-        const long long v = atoll(env);
-        if (v > 0) return v;
-    }
-    return (int64_t)1 << 18;
 }
 
 // Warm-started grids of at least this many column-contiguous columns
@@ -327,13 +289,16 @@ hipError_t launch_cape_only(const CapeGridArgs &a, int math, hipStream_t s)
 // thread's second stream s2, then one counter reset and ascent cover every
 // column.  The copies fill the whole grid's level-major arrays dst (rows of
 // a.ncol; a's profile pointers are those arrays), and each setup pass its
-// part's columns of the records.  In a combined call the winds (hs) are then
-// copied and the helicity launched on s2, after the last setup pass, beside
-// the ascent.  Columns are independent, so the outputs are those of the
-// one-launch call.
+// part's columns of the records.  In a combined call the winds (the first two
+// of wsrc, to a.u and a.v) are then copied and the helicity launched on s2,
+// after the last setup pass, beside the ascent: at these sizes the copies fit
+// under the ascent, and the lane-per-column helicity that reads them ends 1 ms
+// sooner after it than the one that reads the profiles where they lie (2048 x
+// 1024 columns of 137 levels: the step 13.06 ms against 13.68).  Columns are
+// independent, so the outputs are those of the one-launch call.
 hipError_t launch_warm_parts(const CapeGridArgs &a, bool srh, int math, hipStream_t s,
-                             hipStream_t s2, const float *const *src, float *const *dst,
-                             int narr, const HelicityStage *hs)
+                             hipStream_t s2, const float *const *src, float *const *dst, int narr,
+                             const float *const *wsrc, float *const *wdst)
 {
     const int64_t n = a.ncol, nk = a.nk_in, esz = 4;
     int64_t c = (n + WARM_PARTS - 1) / WARM_PARTS;
@@ -403,10 +368,8 @@ hipError_t launch_warm_parts(const CapeGridArgs &a, bool srh, int math, hipStrea
         if ((e = hipEventRecord(setup, s)) != hipSuccess ||
             (e = hipStreamWaitEvent(s2, setup, 0)) != hipSuccess)
             return joined(e);
-        if (hs && (e = launch_transpose_levels(hs->src, hs->dst, hs->narr, hs->n, hs->nk,
-                                               s2)) != hipSuccess)
-            return joined(e);
-        if ((e = launch_cape_grid_accurate(a, false, GRID_SRH, 256, s2)) != hipSuccess)
+        if ((e = launch_transpose_levels(wsrc, wdst, 2, n, nk, s2)) != hipSuccess ||
+            (e = launch_cape_grid_accurate(a, false, GRID_SRH, 256, s2)) != hipSuccess)
             return joined(e);
     }
     CapeGridArgs z = a;
@@ -420,23 +383,34 @@ hipError_t launch_warm_parts(const CapeGridArgs &a, bool srh, int math, hipStrea
 hipError_t run_grid(const CapeGridArgs &a0, bool cape, bool srh, int math, hipStream_t s,
                     float *ext = nullptr, unsigned int *ext_work = nullptr)
 {
-    // float64 inputs (the helicity chain only) are read where they lie
-    const bool stage = a0.ls == 1 && a0.nk_in > 1 && !a0.in_f64;
+    // the helicity chain reads the profiles where they lie
+    const bool stage = cape && a0.ls == 1 && a0.nk_in > 1;
     const bool warm = cape && a0.warm != 0 && math != 2;
-    if (!stage && !warm) return launch_grid(a0, cape, srh, math, s);
+    if (!stage && !warm) return launch_grid(a0, a0, cape, srh, math, s);
     const bool sigma = a0.p != nullptr;
-    const float *src0[5];
+    const float *src0[3];
     int narr = 0;
-    int it = -1, itd = -1, iu = -1, iv = -1, ip = -1;
+    int it = -1, itd = -1, ip = -1;
     if (stage) {
         it = narr; src0[narr++] = a0.t;
         itd = narr; src0[narr++] = a0.td;
         if (sigma) { ip = narr; src0[narr++] = a0.p; }
-        if (srh) { iu = narr; src0[narr++] = a0.u; iv = narr; src0[narr++] = a0.v; }
     }
     const int64_t nk = a0.nk_in;
     const int64_t wfl = warm ? warm_scratch_floats(nk, a0.p_lfc != nullptr) : 0;
-    const int64_t per_col = ((int64_t)narr * nk + wfl) * (int64_t)sizeof(float);
+    // a large warm-started grid: staged in parts, each beside a setup pass
+    hipStream_t s2 = nullptr;
+    bool wparts = false;
+    if (warm && stage && !ext && a0.ncol >= warm_pipe_min_columns() && a0.ncol >= 2 * 64 &&
+        !a0.nk_col && !a0.src_col && !a0.out_index) {
+        s2 = aux_stream();
+        wparts = s2 && s2 != s && thread_event(EV_FORK) && thread_event(EV_JOIN) &&
+                 thread_event(EV_SETUP);
+        for (int i = 1; wparts && i < WARM_PARTS; ++i) wparts = thread_event(EV_PART + i);
+    }
+    // the winds' copies of a combined call in parts
+    const int64_t wind = wparts && srh ? 2 * nk : 0;
+    const int64_t per_col = ((int64_t)narr * nk + wind + wfl) * (int64_t)sizeof(float);
     int64_t chunk = ((int64_t)16 << 30) / per_col;
     if (chunk < ((int64_t)1 << 20)) chunk = (int64_t)1 << 20;
     // XCAPE_STAGE_COLUMNS: columns per chunk, overriding the 16 GiB sizing
@@ -451,98 +425,49 @@ hipError_t run_grid(const CapeGridArgs &a0, bool cape, bool srh, int math, hipSt
         if (chunk > cap) chunk = cap;
     }
     if (chunk > a0.ncol) chunk = a0.ncol;
-    // the helicity-only call in parts (each part's copies in a region of its
-    // own, so that one part's helicity launch can still read them while the
-    // next part is copied), when the whole call fits one chunk's scratch
-    hipStream_t s2 = nullptr;
-    int64_t parts = 1;
-    if (!cape && srh && stage && !ext && chunk >= a0.ncol &&
-        a0.ncol >= srh_pipe_min_columns() && a0.ncol >= 2 * 64 &&
-        (s2 = aux_stream()) != nullptr && s2 != s && thread_event(EV_FORK) &&
-        thread_event(EV_JOIN)) {
-        int64_t c = (a0.ncol + SRH_PARTS - 1) / SRH_PARTS;
-        c = (c + 63) & ~(int64_t)63;   // parts of whole waves
-        chunk = c;
-        parts = (a0.ncol + c - 1) / c;
-    }
-    // a large warm-started grid: staged in parts, each beside a setup pass
-    bool wparts = false;
-    if (warm && stage && !ext && chunk >= a0.ncol && a0.ncol >= warm_pipe_min_columns() &&
-        a0.ncol >= 2 * 64 && !a0.nk_col && !a0.src_col && !a0.out_index) {
-        s2 = aux_stream();
-        wparts = s2 && s2 != s && thread_event(EV_FORK) && thread_event(EV_JOIN) &&
-                 thread_event(EV_SETUP) && thread_event(EV_PART + WARM_PARTS - 1);
-        for (int i = 1; wparts && i < WARM_PARTS; ++i) wparts = thread_event(EV_PART + i);
-    }
+    if (chunk < a0.ncol) wparts = false;
     DevBuf<float> scratch_;
     DevBuf<unsigned int> work_;
     float *scratch = ext;
     unsigned int *work = ext_work;
     hipError_t e = hipSuccess;
     if (!ext) {
-        if ((e = scratch_.alloc((size_t)(narr * nk + wfl) * (size_t)chunk * (size_t)parts,
-                                s)) != hipSuccess)
+        if ((e = scratch_.alloc((size_t)(narr * nk + wind + wfl) * (size_t)chunk, s)) != hipSuccess)
             return e;
         if (warm && (e = work_.alloc(8, s)) != hipSuccess) return e;   // WORK_PARTS counters
         scratch = scratch_.ptr;
         work = work_.ptr;
     }
     const int64_t esz = math == 2 ? 8 : 4;
-    // once a part's helicity launch is on s2, every return joins s2 back into
-    // s first: the scratch is freed on s, and s2 may still read it
-    bool forked = false;
-    const auto joined = [&](hipError_t err) {
-        if (forked) {
-            const hipEvent_t join = thread_event(EV_JOIN);
-            const hipError_t er = hipEventRecord(join, s2);
-            const hipError_t ew = hipStreamWaitEvent(s, join, 0);
-            forked = false;
-            if (err == hipSuccess) err = er != hipSuccess ? er : ew;
-        }
-        return err;
-    };
     for (int64_t c0 = 0; c0 < a0.ncol; c0 += chunk) {
         const int64_t n = chunk < a0.ncol - c0 ? chunk : a0.ncol - c0;
         CapeGridArgs a = a0;
         a.ncol = n;
-        HelicityStage hs_, *hs = nullptr;
-        const float *src[5];
-        float *dst[5];
-        int nfirst = 0;
+        const float *src[3];
+        float *dst[3];
         if (stage) {
             const int64_t o = c0 * nk;
-            // (parts > 1: the part's own region)
-            float *cs = scratch + (parts > 1 ? (size_t)narr * (size_t)nk * (size_t)c0 : 0);
             for (int i = 0; i < narr; ++i) {
                 src[i] = src0[i] + o;
-                dst[i] = cs + (size_t)i * (size_t)nk * (size_t)n;
+                dst[i] = scratch + (size_t)i * (size_t)nk * (size_t)n;
             }
-            // in a combined call the winds are copied on the helicity's stream,
-            // beside the CAPE launches; a grid in parts is copied part by part
-            nfirst = cape && srh ? narr - 2 : narr;
-            if (!wparts && (e = launch_transpose_levels(src, dst, nfirst, n, nk, s)) !=
-                               hipSuccess)
-                return joined(e);
-            if (nfirst < narr) {
-                hs_ = HelicityStage{{src[iu], src[iv]}, {dst[iu], dst[iv]}, 2, n, nk};
-                hs = &hs_;
-            }
+            // a grid in parts is copied part by part
+            if (!wparts && (e = launch_transpose_levels(src, dst, narr, n, nk, s)) != hipSuccess)
+                return e;
             a.ls = n;
             a.t = dst[it];
             a.td = dst[itd];
             if (sigma) a.p = dst[ip];
-            if (srh) { a.u = dst[iu]; a.v = dst[iv]; }
         } else {
             // level-major input (or a single level): the chunk's columns
             // start c0 into each level's row
             a.t += c0; a.td += c0;
             if (sigma) a.p += c0;
-            if (srh) { a.u += c0; a.v += c0; }
         }
         a.ps += c0; a.ts += c0; a.tds += c0;
         if (a.start) a.start += c0;
         if (warm) {
-            float *w = scratch + (size_t)narr * (size_t)nk * (size_t)n;
+            float *w = scratch + (size_t)(narr * nk + wind) * (size_t)n;
             const size_t lv = (size_t)(nk + 1) * (size_t)n;
             a.env = w;
             a.par = w + 4 * lv;
@@ -569,22 +494,26 @@ hipError_t run_grid(const CapeGridArgs &a0, bool cape, bool srh, int math, hipSt
                 a.mean6 = static_cast<char *>(a.mean6) + b;
             }
         }
-        if (parts > 1) {
-            // this part's helicity on s2, once its copies are done; the next
-            // part's copies go on s meanwhile
-            const hipEvent_t fork = thread_event(EV_FORK);
-            if ((e = hipEventRecord(fork, s)) == hipSuccess &&
-                (e = hipStreamWaitEvent(s2, fork, 0)) == hipSuccess) {
-                forked = true;
-                e = launch_cape_grid_accurate(a, math == 2, GRID_SRH, 256, s2);
-            }
-            // after the last part, or a failed one: s waits for s2
-            if (e != hipSuccess || c0 + n >= a0.ncol) e = joined(e);
-            if (e != hipSuccess) return e;
-            continue;
+        CapeGridArgs h = a;
+        if (srh) {
+            // (column c's level k at c * nk + k, or k * ls + c)
+            const int64_t o = a0.ls == 1 ? c0 * nk : c0;
+            h.ls = a0.ls;
+            h.t = a0.t + o;
+            h.td = a0.td + o;
+            if (sigma) h.p = a0.p + o;
+            h.u = a0.u + o;
+            h.v = a0.v + o;
         }
-        if (wparts) e = launch_warm_parts(a, srh, math, s, s2, src, dst, nfirst, hs);
-        else e = launch_grid(a, cape, srh, math, s, hs);
+        if (wparts) {
+            const float *wsrc[2] = {h.u, h.v};
+            float *wdst[2] = {scratch + (size_t)narr * (size_t)nk * (size_t)n,
+                              scratch + (size_t)(narr + 1) * (size_t)nk * (size_t)n};
+            if (srh) { a.u = wdst[0]; a.v = wdst[1]; }
+            e = launch_warm_parts(a, srh, math, s, s2, src, dst, narr, wsrc, wdst);
+        } else {
+            e = launch_grid(a, h, cape, srh, math, s);
+        }
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -888,7 +817,7 @@ int stream_host_grid(const GridCall &c, const CapeGridArgs &tmpl, bool want_cape
     CapeGridArgs shape = tmpl;   // the chunks' launches read column-contiguous profiles
     shape.ls = 1;
     shape.p = c.p_shared ? nullptr : c.p;
-    const size_t scr_bytes = align_up((size_t)grid_scratch_floats(shape, want_cape, want_srh, math) *
+    const size_t scr_bytes = align_up((size_t)grid_scratch_floats(shape, want_cape, math) *
                                       (size_t)m * sizeof(float));
     const size_t slot_bytes = in_bytes + out_bytes + scr_bytes + STAGE_ALIGN;   // + work counters
     const size_t shared = align_up((size_t)nk * sizeof(float)) +
@@ -1137,7 +1066,7 @@ int grid_entry(const GridCall &c)
     if (c.noalloc) {
         // the whole call's scratch in the caller-independent array: the
         // warm ascent's counters first, then the staged profiles and records
-        const size_t per = (size_t)grid_scratch_floats(a, true, false, math) * sizeof(float);
+        const size_t per = (size_t)grid_scratch_floats(a, true, math) * sizeof(float);
         const size_t need = NOALLOC_HEAD + per * (size_t)c.ncol;
         if (need > NOALLOC_SCRATCH_BYTES)
             return fail(XCAPE_EINVAL,

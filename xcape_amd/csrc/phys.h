@@ -223,10 +223,12 @@ __device__ __forceinline__ double xc_sconst(double c)
 // hardware reciprocal refined by two Newton steps (s enters only the
 // correction term).  Within an ulp of ln x for positive finite x (the
 // hardware's frexp normalises subnormals); ln 0 = -inf, ln inf = inf, and
-// NaN for negative x or NaN, as the C library's.
+// NaN for negative x or NaN, as the C library's.  CHECKED: the caller makes
+// sure that x is positive and finite.
+template <bool CHECKED = false>
 __device__ __forceinline__ double log_core_f64(double x)
 {
-    if (__builtin_expect(!(x > 0.0 && x <= 0x1.fffffffffffffp+1023), 0))
+    if (!CHECKED && __builtin_expect(!(x > 0.0 && x <= 0x1.fffffffffffffp+1023), 0))
         return x == 0.0 ? -__builtin_inf() : (x > 0.0 ? x : __builtin_nan(""));
     constexpr double LN2_HI = 0x1.62e42fe000000p-1;
     constexpr double LN2_LO = 0x1.f473de6af278fp-30;
@@ -267,9 +269,11 @@ __device__ __forceinline__ double log_core_f64(double x)
 // below 4e-19), scaled by 2^k.  Within an ulp of e^x wherever the result
 // is normal (-708.3 < x < 709.7); subnormal results, overflow to inf,
 // underflow to 0, NaN as the C library's (up to an ulp of the subnormal).
+// CHECKED: as above, for x within (-745.2, 709.8).
+template <bool CHECKED = false>
 __device__ __forceinline__ double exp_core_f64(double x)
 {
-    if (__builtin_expect(!(x > -745.2 && x < 709.8), 0))
+    if (!CHECKED && __builtin_expect(!(x > -745.2 && x < 709.8), 0))
         return x != x ? x : (x > 0.0 ? __builtin_inf() : 0.0);
     constexpr double INV_LN2 = 0x1.71547652b82fep+0;
     constexpr double LN2_HI = 0x1.62e42fe000000p-1;
