@@ -105,6 +105,29 @@ def test_streamed_pressure_levels(hip, monkeypatch, start):
           hip.srh(*dw, p_shared=True, start_lev=dst))
 
 
+@pytest.mark.parametrize('ncol,chunk_mb', [(1, None), (37, '1'), (5000, None), (5000, '1')])
+def test_streamed_double_winds(hip, monkeypatch, ncol, chunk_mb):
+    """float64 profiles of a helicity call: 2432 bytes per column, so 1 MB
+    chunks are 384 columns (128, 192, then 384) and 5000 columns take fifteen;
+    the device call is the reference, equal bit for bit."""
+    if chunk_mb is None:
+        monkeypatch.delenv('XCAPE_HOST_CHUNK_MB', raising=False)
+    else:
+        monkeypatch.setenv('XCAPE_HOST_CHUNK_MB', chunk_mb)
+    _, args = _sigma(ncol, 6)
+    args = [np.asarray(a, np.float64) for a in args]
+    for motions in (False, True):
+        kw = dict(fp64=True, inputs_f64=True, motions=motions)
+        _same(hip.srh(*args, **kw), hip.srh(*_dev(args), **kw))
+    c = synthetic.pressure_columns(ncol, 78, winds=True)
+    args = [np.asarray(c[k], np.float64)
+            for k in ('p', 't', 'td', 'u', 'v', 'ps', 'ts', 'tds', 'us', 'vs')]
+    st = (1 + np.arange(ncol) % 3).astype(np.int32)
+    kw = dict(fp64=True, inputs_f64=True, p_shared=True)
+    _same(hip.srh(*args, start_lev=st, **kw),
+          hip.srh(*_dev(args), start_lev=_dev([st])[0], **kw))
+
+
 def test_streamed_srh_and_fused(hip, monkeypatch):
     """The fused call's 1216 bytes of input per column: 832-column chunks
     (the first two of 256 and 448 columns), eight of them for 5000 columns,

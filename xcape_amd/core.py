@@ -97,7 +97,7 @@ def _any_dask_array(*args):
 def pressure_start_levels(p1d, ps):
     """1-based first level with p <= ps for each column (core.py:286-289)."""
     tmp = ps[None, :] - p1d[:, None]
-    return (np.ma.masked_less(tmp, 0).argmin(axis=0) + 1).astype(np.int32)
+    return (np.where(tmp < 0, np.inf, tmp).argmin(axis=0) + 1).astype(np.int32)
 
 
 def calc_cape(*args, **kwargs):

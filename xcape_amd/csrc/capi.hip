@@ -557,14 +557,25 @@ struct GridCall {
 //     area each) run the chunk's kernels once its upload has ended, download
 //     its outputs, and are drained into the caller's arrays when the calling
 //     thread comes back to the slot.
-// The first chunks are a quarter and a half of the others, so the first
-// upload starts early.  A chunk of an array is one contiguous range of the
-// caller's array and one contiguous run of the staging areas: a chunk moves
-// in one upload and one download.
+// A call of up to STAGE_WHOLE_MB of input goes as one chunk.  An ascent's
+// kernel takes 0.6 to 1.4 ms for few columns as for a device full, longer than
+// such an upload, and chunks whose streams share a hardware queue wait for each
+// other.  In one chunk / a quarter, a half and the rest (median us, 8 threads):
+// 40 levels, surface, 2 MB 688 / 1635, 24 MB 1365 / 1792, 64 MB 2900 / 2994,
+// 107 MB 4198 / 3526; 137 levels, most unstable, pseudo-ice, 2 MB 1246 / 2222,
+// 24 MB 2222 / 3602, 64 MB 3127 / 4436, 107 MB 4883 / 4737.  Larger calls start
+// with a quarter and a half of a chunk, so that the first upload and the first
+// kernels start early.  A chunk of an array is one contiguous range of the
+// caller's array and one contiguous run of the staging areas.
 
 constexpr int STAGE_IN = 3;
 constexpr int STAGE_SLOTS = 4;
 constexpr int STAGE_SETS = 2;   // at most this many calls stream at once; others wait
+constexpr size_t STAGE_WHOLE_MB = 64;
+// bytes of a chunk that goes in one upload; the arrays of a larger one go one by
+// one, each while the next is copied (64 MB in one chunk, 40 levels: 2900 us
+// against 3152; 137 levels: 3127 against 3400)
+constexpr size_t STAGE_ONE_UPLOAD = (size_t)2 << 20;
 constexpr size_t STAGE_ALIGN = 256;
 
 size_t align_up(size_t x) { return (x + STAGE_ALIGN - 1) / STAGE_ALIGN * STAGE_ALIGN; }
@@ -577,19 +588,22 @@ struct Slab {
     const char *src[12];   // inputs: the caller's arrays
     char *dst[12];         // outputs: the caller's arrays
     size_t cb[12];         // bytes per column
-    int add(const void *in, void *out, size_t col_bytes)
+    size_t whole[12];      // or bytes of an array that goes with every chunk
+    int add(const void *in, void *out, size_t col_bytes, size_t whole_bytes = 0)
     {
         src[count] = static_cast<const char *>(in);
         dst[count] = static_cast<char *>(out);
         cb[count] = col_bytes;
+        whole[count] = whole_bytes;
         return count++;
     }
+    size_t bytes(int i, int64_t n) const { return whole[i] + (size_t)n * cb[i]; }
     size_t place(int64_t n, size_t *off) const
     {
         size_t at = 0;
         for (int i = 0; i < count; ++i) {
             off[i] = at;
-            at = align_up(at + (size_t)n * cb[i]);
+            at = align_up(at + bytes(i, n));
         }
         return at;
     }
@@ -771,19 +785,20 @@ int stream_host_grid(const GridCall &c, const CapeGridArgs &tmpl, bool want_cape
 {
     const int64_t nk = c.nk, ncol = c.ncol;
     const size_t osz = c.fp64 ? sizeof(double) : sizeof(float);
-    const size_t prof = (size_t)nk * sizeof(float);
+    const size_t isz = tmpl.in_f64 ? sizeof(double) : sizeof(float);
+    const size_t prof = (size_t)nk * isz;
     Slab in, out;
     const int i_t = in.add(c.t, nullptr, prof), i_td = in.add(c.td, nullptr, prof);
-    const int i_p = c.p_shared ? -1 : in.add(c.p, nullptr, prof);
-    const int i_ps = in.add(c.ps, nullptr, 4), i_ts = in.add(c.ts, nullptr, 4);
-    const int i_tds = in.add(c.tds, nullptr, 4);
+    const int i_p = c.p_shared ? in.add(c.p, nullptr, 0, prof) : in.add(c.p, nullptr, prof);
+    const int i_ps = in.add(c.ps, nullptr, isz), i_ts = in.add(c.ts, nullptr, isz);
+    const int i_tds = in.add(c.tds, nullptr, isz);
     const int i_st = c.start ? in.add(c.start, nullptr, 4) : -1;
     int i_u = -1, i_v = -1, i_us = -1, i_vs = -1;
     if (want_srh) {
         i_u = in.add(c.u, nullptr, prof);
         i_v = in.add(c.v, nullptr, prof);
-        i_us = in.add(c.us, nullptr, 4);
-        i_vs = in.add(c.vs, nullptr, 4);
+        i_us = in.add(c.us, nullptr, isz);
+        i_vs = in.add(c.vs, nullptr, isz);
     }
     int o_cape = -1, o_cin = -1, o_z = -1, o_mul = -1, o_lfc = -1, o_el = -1;
     int o_srm = -1, o_slm = -1, o_rm = -1, o_lm = -1, o_mw = -1;
@@ -811,6 +826,7 @@ int stream_host_grid(const GridCall &c, const CapeGridArgs &tmpl, bool want_cape
     // columns per chunk: about XCAPE_HOST_CHUNK_MB of input, a multiple of 64
     int64_t m = ((int64_t)host_chunk_mb() << 20) / (int64_t)in_col / 64 * 64;
     if (m < 64) m = 64;
+    const bool whole = (size_t)ncol * in_col <= (STAGE_WHOLE_MB << 20) && m >= ncol;
     if (m > ncol) m = ncol;
     size_t off_in[12], off_out[12];
     const size_t in_bytes = in.place(m, off_in), out_bytes = out.place(m, off_out);
@@ -820,40 +836,39 @@ int stream_host_grid(const GridCall &c, const CapeGridArgs &tmpl, bool want_cape
     const size_t scr_bytes = align_up((size_t)grid_scratch_floats(shape, want_cape, math) *
                                       (size_t)m * sizeof(float));
     const size_t slot_bytes = in_bytes + out_bytes + scr_bytes + STAGE_ALIGN;   // + work counters
-    const size_t shared = align_up((size_t)nk * sizeof(float)) +
-                          align_up(ST_COUNT * sizeof(unsigned long long));
+    const size_t shared = align_up(ST_COUNT * sizeof(unsigned long long));
     int dv = 0;
     hipError_t e = hipGetDevice(&dv);
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
     if (c.stream && (e = hipStreamSynchronize((hipStream_t)c.stream)) != hipSuccess)
         return hip_fail(e, "hipStreamSynchronize(stream)");
     StagingSet *st = acquire_staging(dv);
-    struct Finish {   // on every return: the set's streams drained, the set back in the pool
+    // on every return: the set back in the pool, its streams drained first
+    // (every chunk waited for already, unless the call ends early)
+    struct Finish {
         StagingSet *st;
+        bool drained;
         ~Finish()
         {
-            if (st->up) (void)hipStreamSynchronize(st->up);
-            for (int i = 0; i < STAGE_SLOTS; ++i)
-                if (st->stream[i]) (void)hipStreamSynchronize(st->stream[i]);
+            if (!drained) {
+                if (st->up) (void)hipStreamSynchronize(st->up);
+                for (int i = 0; i < STAGE_SLOTS; ++i)
+                    if (st->stream[i]) (void)hipStreamSynchronize(st->stream[i]);
+            }
             release_staging(st);
         }
-    } finish{st};
+    } finish{st, false};
     if ((e = st->reserve(dv, in_bytes, out_bytes, shared + STAGE_SLOTS * slot_bytes)))
         return hip_fail(e, "pinned staging allocation");
-    char *const p1d = st->dev;
-    unsigned long long *const dstats =
-        reinterpret_cast<unsigned long long *>(st->dev + align_up((size_t)nk * sizeof(float)));
+    unsigned long long *const dstats = reinterpret_cast<unsigned long long *>(st->dev);
 #define XC_TRY(x) if ((e = (x)) != hipSuccess) return hip_fail(e, #x)
-    if (c.p_shared)
-        XC_TRY(hipMemcpyAsync(p1d, c.p, (size_t)nk * sizeof(float), hipMemcpyHostToDevice, st->up));
+    // (ahead of the first chunk's `uploaded`, which its kernels wait for)
     if (c.stats && want_cape) XC_TRY(zero_counters(dstats, ST_COUNT, st->up));
-    XC_TRY(hipStreamSynchronize(st->up));
     struct Pending {
         int64_t c0 = 0, n = 0;
         bool busy = false;
     } pend[STAGE_SLOTS];
     bool in_used[STAGE_IN] = {};
-    CopyJob jobs[12];
     const int threads = host_threads();
     int64_t chunk_no = 0;
     // the outputs of the chunk that slot sl last ran, into the caller's arrays
@@ -861,10 +876,11 @@ int stream_host_grid(const GridCall &c, const CapeGridArgs &tmpl, bool want_cape
         const hipError_t r = hipEventSynchronize(st->done[sl]);
         if (r != hipSuccess) return r;
         size_t off[12];
+        CopyJob jobs[12];
         out.place(pend[sl].n, off);
         for (int i = 0; i < out.count; ++i)
             jobs[i] = {out.dst[i] + (size_t)pend[sl].c0 * out.cb[i], st->pin_out[sl] + off[i],
-                       (size_t)pend[sl].n * out.cb[i]};
+                       out.bytes(i, pend[sl].n)};
         parallel_copy(jobs, out.count, threads);
         pend[sl].busy = false;
         return hipSuccess;
@@ -872,25 +888,39 @@ int stream_host_grid(const GridCall &c, const CapeGridArgs &tmpl, bool want_cape
     for (int64_t c0 = 0, n = 0; c0 < ncol; c0 += n, ++chunk_no) {
         const int r = (int)(chunk_no % STAGE_IN), sl = (int)(chunk_no % STAGE_SLOTS);
         // a quarter, a half, then whole chunks
-        n = chunk_no >= 2 ? m : ((m >> (2 - chunk_no)) + 63) / 64 * 64;
+        n = whole || chunk_no >= 2 ? m : ((m >> (2 - chunk_no)) + 63) / 64 * 64;
         if (n < 64) n = 64;
         if (n > m) n = m;
         if (n > ncol - c0) n = ncol - c0;
         if (in_used[r]) XC_TRY(hipEventSynchronize(st->uploaded[r]));
         size_t oi[12], oo[12];
+        CopyJob jobs[12];
         const size_t ib = in.place(n, oi), ob = out.place(n, oo);
         for (int i = 0; i < in.count; ++i)
-            jobs[i] = {st->pin_in[r] + oi[i], in.src[i] + (size_t)c0 * in.cb[i],
-                       (size_t)n * in.cb[i]};
-        parallel_copy(jobs, in.count, threads);
-        // the slot's device buffers are free once its previous chunk is done
-        if (pend[sl].busy) XC_TRY(drain(sl));
+            jobs[i] = {st->pin_in[r] + oi[i], in.src[i] + (size_t)c0 * in.cb[i], in.bytes(i, n)};
         char *din = st->dev + shared + (size_t)sl * slot_bytes;
         char *dout = din + in_bytes;
         float *dscr = reinterpret_cast<float *>(dout + out_bytes);
         unsigned int *dwork = reinterpret_cast<unsigned int *>(dout + out_bytes + scr_bytes);
         hipStream_t ss = st->stream[sl];
-        XC_TRY(hipMemcpyAsync(din, st->pin_in[r], ib, hipMemcpyHostToDevice, st->up));
+        if (ib <= STAGE_ONE_UPLOAD) {
+            parallel_copy(jobs, in.count, threads);
+            // the slot's device buffers are free once its previous chunk is done
+            if (pend[sl].busy) XC_TRY(drain(sl));
+            XC_TRY(hipMemcpyAsync(din, st->pin_in[r], ib, hipMemcpyHostToDevice, st->up));
+        } else {
+            // each profile array by itself, the small ones between them together
+            for (int i = 0, e1; i < in.count; i = e1) {
+                e1 = i + 1;
+                if (in.cb[i] != prof)
+                    while (e1 < in.count && in.cb[e1] != prof) ++e1;
+                parallel_copy(jobs + i, e1 - i, threads);
+                if (i == 0 && pend[sl].busy) XC_TRY(drain(sl));
+                const size_t end = e1 < in.count ? oi[e1] : ib;
+                XC_TRY(hipMemcpyAsync(din + oi[i], st->pin_in[r] + oi[i], end - oi[i],
+                                      hipMemcpyHostToDevice, st->up));
+            }
+        }
         XC_TRY(hipEventRecord(st->uploaded[r], st->up));
         in_used[r] = true;
         XC_TRY(hipStreamWaitEvent(ss, st->uploaded[r], 0));
@@ -901,7 +931,7 @@ int stream_host_grid(const GridCall &c, const CapeGridArgs &tmpl, bool want_cape
         a.ls = 1;
         a.t = fin(i_t); a.td = fin(i_td);
         a.p = c.p_shared ? nullptr : fin(i_p);
-        a.p1d = c.p_shared ? reinterpret_cast<const float *>(p1d) : nullptr;
+        a.p1d = c.p_shared ? fin(i_p) : nullptr;
         a.start = reinterpret_cast<const int32_t *>(fin(i_st));
         a.ps = fin(i_ps); a.ts = fin(i_ts); a.tds = fin(i_tds);
         a.u = fin(i_u); a.v = fin(i_v); a.us = fin(i_us); a.vs = fin(i_vs);
@@ -928,6 +958,7 @@ int stream_host_grid(const GridCall &c, const CapeGridArgs &tmpl, bool want_cape
         copy_stats(h, c.stats);
     }
 #undef XC_TRY
+    finish.drained = true;
     return XCAPE_OK;
 }
 
@@ -1006,7 +1037,7 @@ int grid_entry(const GridCall &c)
     const int math = c.fp64 ? 2 : ((c.flags & XCAPE_FAST_MATH) ? 1 : 0);
     // host arrays in column order stream through pinned staging; level-major
     // host arrays go whole through stream-ordered buffers
-    if (!dev && !(c.flags & XCAPE_LEVEL_MAJOR) && !f64in)
+    if (!dev && !(c.flags & XCAPE_LEVEL_MAJOR))
         return stream_host_grid(c, a, want_cape, want_srh, math);
     // input floats per element (double inputs: two)
     const size_t iw = f64in ? 2 : 1;
