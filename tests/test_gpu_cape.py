@@ -613,6 +613,22 @@ def test_warm_parts_match_one_launch(hip, monkeypatch):
     assert got[0][-1]['columns'] == 3000
 
 
+@pytest.mark.parametrize('levels', [False, True])
+@pytest.mark.parametrize('ncol', [1, 2, 65, 1023, 1025, 5000, 33000])
+def test_warm_small_launches_match_the_large(hip, ncol, levels):
+    """A warm ascent of fewer columns than the device has lanes spreads them
+    over its waves, a few to each; a column's result does not depend on it."""
+    import torch
+    c = synthetic.sigma_columns(70000, 24, 19)
+    args = [torch.from_numpy(np.ascontiguousarray(c[k])).cuda()
+            for k in ('p', 't', 'td', 'ps', 'ts', 'tds')]
+    kw = dict(pinc=700., source=2, adiabat=3, warm_start=True, levels=levels)
+    whole = hip.cape(*args, **kw)
+    part = hip.cape(*(a[:ncol] for a in args), **kw)
+    for w, p in zip(whole, part):
+        np.testing.assert_array_equal(p.cpu().numpy(), w[:ncol].cpu().numpy())
+
+
 @pytest.mark.parametrize('adiabat', [1, 2, 3, 4])
 @pytest.mark.parametrize('ncol,nk', [(1, 60), (63, 40), (1024, 40), (1025, 33), (2111, 40),
                                      (65537, 24), (131072, 20), (131073, 20)])

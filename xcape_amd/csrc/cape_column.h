@@ -51,6 +51,18 @@ XC_HD __forceinline__ void xc_opaque(int &v)
 #endif
 }
 
+// v in a register of its own from here on (a value loaded from memory has
+// arrived, a copy has been made); no code on the host.
+template <typename V>
+XC_HD __forceinline__ void xc_arrived(V &v)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    __asm__ volatile("" : "+v"(v));
+#else
+    (void)v;
+#endif
+}
+
 template <typename T> struct ColumnOut {
     T cape, cin, zout;
     int mulvl;
@@ -1019,7 +1031,13 @@ struct WarmAscent {
             if constexpr (LEVELS) pb = e_p;
             Level<T> lv;
             if constexpr (HasEnv<C>::value) {
-                lv = level_unpack(nx, nx_p);
+                // (copied before the load, so that the load can go to nx's
+                // own registers and nothing waits for it before the next level)
+                LevelRec r = nx;
+                T rp = nx_p;
+                xc_arrived(r.dp); xc_arrived(r.pi); xc_arrived(r.thv); xc_arrived(r.meta);
+                if constexpr (LEVELS) xc_arrived(rp);
+                lv = level_unpack(r, rp);
                 if (k + 1 < nk) {
                     nx = col.rec_at(k + 1);
                     if constexpr (LEVELS) nx_p = col.p_at(k + 1);

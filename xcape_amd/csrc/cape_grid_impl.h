@@ -423,10 +423,11 @@ warm_setup_kernel(CapeGridArgs a)
 // Workgroups are dispatched to the eight XCDs in turn, so the waves of part
 // blockIdx % 8 all run on one XCD.  (Every part holds an equal share of the
 // columns and as many waves, so the parts drain together.)  A wave takes its
-// part's columns 64 at a time (one atomic per 64 columns); its lanes draw
-// from that block as they finish their columns.
+// part's columns cpw at a time, one for each of its first cpw lanes (one atomic
+// per cpw columns); the lanes draw from that block as they finish their
+// columns, and lane l >= cpw repeats lane l % cpw's.
 constexpr uint32_t WORK_PARTS = 8;
-constexpr uint32_t WORK_BLOCK = 64;
+
 
 __device__ __forceinline__ uint32_t work_part_begin(uint32_t ncol, uint32_t part,
                                                     uint32_t parts)
@@ -446,7 +447,7 @@ __host__ __device__ __forceinline__ uint32_t work_parts(uint32_t grid)
 // scalar registers to VGPR lanes and shuffled more (7 waves ran 1.5 % faster).
 template <bool ICE, bool PSEUDO, bool PREDICT, bool STATS, bool LEVELS = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7)))
-warm_ascent_kernel(CapeGridArgs a)
+warm_ascent_kernel(CapeGridArgs a, int cpw)
 {
     using T = float;
     const uint32_t ncol = (uint32_t)a.ncol;
@@ -454,37 +455,44 @@ warm_ascent_kernel(CapeGridArgs a)
       *zout = static_cast<T *>(a.zout);
     const float4 *recs = reinterpret_cast<const float4 *>(a.par);
     const int lane = threadIdx.x & 63;
-    const uint64_t below = (1ull << lane) - 1ull;
+    const uint32_t slot = (uint32_t)lane % (uint32_t)cpw;
+    const uint64_t slots = ~0ull >> (64 - cpw), below = (1ull << slot) - 1ull;
     WarmAscent<T, XC_MATH, ICE, PSEUDO, LEVELS> w;
     LaneStats st;
     uint32_t col = 0;
     bool have = false, need = true;
     // wave-uniform: the wave's part (its XCD's), its current block of columns
-    // [blk, blk + 64) and the block's slots handed out
+    // [blk, blk + cpw) and how many of them are handed out
     const uint32_t parts = work_parts(gridDim.x);
     const uint32_t part = blockIdx.x % parts;
     const uint32_t part_end = work_part_begin(ncol, part + 1, parts);
-    uint32_t blk = 0, used = WORK_BLOCK;
+    const uint32_t block = (uint32_t)cpw;
+    uint32_t blk = 0, used = block;
     bool drained = false;
     for (;;) {
-        const uint64_t want = __ballot(need);
+        const uint64_t want = __ballot(need) & slots;
         if (want != 0 && !drained) {
-            if (used >= WORK_BLOCK) {
+            if (used >= block) {
                 uint32_t b = 0;
-                if (lane == 0) b = atomicAdd(a.work + part, WORK_BLOCK);
+                if (lane == 0) b = atomicAdd(a.work + part, block);
                 blk = __builtin_amdgcn_readfirstlane(b);
                 used = 0;
                 drained = blk >= part_end;
             }
             if (!drained) {
-                uint32_t avail = WORK_BLOCK - used;
+                uint32_t avail = block - used;
                 if (blk + used + avail > part_end) avail = part_end - blk - used;
                 const uint32_t rank = (uint32_t)__popcll(want & below);
                 if (need && rank < avail) {
                     col = blk + used + rank;
                     need = false;
-                    const float4 r0 = recs[4 * col], r1 = recs[4 * col + 1],
-                                 r2 = recs[4 * col + 2], r3 = recs[4 * col + 3];
+                    float4 r0 = recs[4 * col], r1 = recs[4 * col + 1],
+                           r2 = recs[4 * col + 2], r3 = recs[4 * col + 3];
+                    // (all here before the trips' loads: a later wait for one
+                    // of these would wait for the next level's record too)
+                    for (float4 *r : {&r0, &r1, &r2, &r3}) {
+                        xc_arrived(r->x); xc_arrived(r->y); xc_arrived(r->z); xc_arrived(r->w);
+                    }
                     const int kmax = __float_as_int(r0.x);
                     if (kmax >= 0) {
                         Parcel<T> pc;
@@ -507,7 +515,7 @@ warm_ascent_kernel(CapeGridArgs a)
                     need = !have;
                 }
                 const uint32_t got = (uint32_t)__popcll(want);
-                used = avail == 0 ? WORK_BLOCK : used + (got < avail ? got : avail);
+                used = avail == 0 ? block : used + (got < avail ? got : avail);
             }
         }
         // the wave ends when every lane has run out of columns
@@ -522,15 +530,17 @@ warm_ascent_kernel(CapeGridArgs a)
                 for (int b = 0; b < 6; ++b) st.blk_lanes[b] += (st.blocks >> b) & 1u;
             }
             if (done) {
-                ColumnOut<T> o;
-                w.result(o);
-                const int64_t oc = out_col(a, col);
-                cape[oc] = o.cape;
-                cin[oc] = o.cin;
-                zout[oc] = o.zout;
-                if constexpr (LEVELS) {
-                    static_cast<float *>(a.p_lfc)[oc] = o.p_lfc;
-                    static_cast<float *>(a.p_el)[oc] = o.p_el;
+                if (lane < cpw) {
+                    ColumnOut<T> o;
+                    w.result(o);
+                    const int64_t oc = out_col(a, col);
+                    cape[oc] = o.cape;
+                    cin[oc] = o.cin;
+                    zout[oc] = o.zout;
+                    if constexpr (LEVELS) {
+                        static_cast<float *>(a.p_lfc)[oc] = o.p_lfc;
+                        static_cast<float *>(a.p_el)[oc] = o.p_el;
+                    }
                 }
                 have = false;
                 need = true;
@@ -672,15 +682,25 @@ hipError_t launch_cape(const CapeGridArgs &a, int block, hipStream_t s)
                 : launch_cape_f<T, uint64_t, false, false>(a, block, s);
 }
 
-// Blocks of the persistent ascent: as many as the device holds at once, never
-// more than the columns need (occupancy queried once per instantiation and
-// block size)
+// Blocks of the persistent ascent and the columns a wave has in flight (*cpw):
+// as many blocks as the device holds at once, never more than the columns need
+// (occupancy queried once per instantiation and block size).
+//
+// A launch of fewer columns than the SIMDs have lanes puts a wave on each SIMD
+// and shares the columns out: a wave runs a block of the trip whenever one of
+// its columns is there, so fewer columns are fewer blocks, and the lanes
+// without a column repeat one (a wave with few active lanes runs slower than a
+// full one).  121 x 97 columns of 50 levels, pseudo-ice: 1030 us 64 to a wave,
+// 922 with 12; 1024 columns: 982 us and 698 with one; more waves than SIMDs are
+// slower again (65 536 columns of 137 levels: 859 us, 988 with 32).  The
+// counted launches take 64, so that no column is counted twice.
 template <bool ICE, bool PSEUDO, bool PREDICT, bool STATS, bool LEVELS>
-int ascent_grid(int block, int64_t ncol)
+int ascent_grid(int block, int64_t ncol, int *cpw)
 {
     static int per_cu[5] = {-1, -1, -1, -1, -1};   // by block / 64
     static int ncu = 0;
     const int slot = block / 64;
+    *cpw = 64;
     if (slot < 1 || slot > 4) return 1;
     if (per_cu[slot] < 0) {
         int dev = 0, pc = 0;
@@ -694,11 +714,17 @@ int ascent_grid(int block, int64_t ncol)
             pc = 1;
         per_cu[slot] = pc;
     }
-    const int64_t need = (ncol + block - 1) / block;
-    const int64_t full = (int64_t)(ncu > 0 ? ncu : 1) * per_cu[slot];
-    int64_t g = need < full ? need : full;
-    // a multiple of the work parts, so that every part has as many waves
-    if (g >= (int64_t)WORK_PARTS) g -= g % WORK_PARTS;
+    const int64_t cus = ncu > 0 ? ncu : 1, simds = 4 * cus;
+    if (!STATS && ncol < 64 * simds) *cpw = (int)((ncol + simds - 1) / simds);
+    const int64_t cols = (int64_t)*cpw * slot;   // a block's columns
+    int64_t g = (ncol + cols - 1) / cols;
+    // a multiple of the work parts, so that every part has as many waves:
+    // rounded up, since one column too many for a part's waves is a second
+    // ascent for one of them (121 x 97 columns: 1526 us with 40 blocks, 1030
+    // with 48)
+    if (g > (int64_t)WORK_PARTS) g = (g + WORK_PARTS - 1) / WORK_PARTS * WORK_PARTS;
+    const int64_t full = cus * per_cu[slot];
+    if (g > full) g = full >= (int64_t)WORK_PARTS ? full - full % WORK_PARTS : full;
     return (int)g;
 }
 
@@ -716,11 +742,12 @@ hipError_t launch_warm_s(const CapeGridArgs &a, int block, hipStream_t s)
             return e;
         if (a.warm_phase == 1) return hipSuccess;
     }
-    const int grid = ascent_grid<ICE, PSEUDO, PREDICT, STATS, LEVELS>(block, a.ncol);
+    int cpw = 64;
+    const int grid = ascent_grid<ICE, PSEUDO, PREDICT, STATS, LEVELS>(block, a.ncol, &cpw);
     // the counters start at their parts' first columns, for the grid's parts
     warm_reset_kernel<<<1, 64, 0, s>>>(a.work, (uint32_t)a.ncol, (uint32_t)grid);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    warm_ascent_kernel<ICE, PSEUDO, PREDICT, STATS, LEVELS><<<grid, block, 0, s>>>(a);
+    warm_ascent_kernel<ICE, PSEUDO, PREDICT, STATS, LEVELS><<<grid, block, 0, s>>>(a, cpw);
     return hipGetLastError();
 }
 
