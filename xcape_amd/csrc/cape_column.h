@@ -36,11 +36,6 @@ namespace xcape {
 
 enum { SRC_SURFACE = 1, SRC_MU = 2, SRC_ML = 3 };
 
-// Fixed-point iterations per trip of the warm-started loop.
-#ifndef XC_ITERS_PER_TRIP
-#define XC_ITERS_PER_TRIP 2
-#endif
-
 // Makes v's value unknown to the optimiser at this point (no code).
 XC_HD __forceinline__ void xc_opaque(int &v)
 {
@@ -874,7 +869,7 @@ XC_HD void cape_column(const C &col, int nk, T pinc, int source, T ml_depth,
 //
 // Loop shape: with one or two iterations per sub-step the wavefront would
 // spend most of its time waiting for the lane with the most iterations if
-// sub-steps were lock-stepped.  Here every trip does up to XC_ITERS_PER_TRIP
+// sub-steps were lock-stepped.  Here every trip does up to two
 // iterations for every running lane, and each lane moves to its next sub-step
 // or level on its own (the set-up blocks execute under the mask of the lanes
 // that need them).
@@ -923,17 +918,23 @@ XC_HD __forceinline__ T adiabat_shape(T t, T p, T th, bool ice)
 
 template <typename T, int MATH, bool ICE, bool PSEUDO, bool LEVELS = false>
 struct WarmAscent {
-    enum { M_LEVEL = 0, M_SUB = 1, M_ITER = 2, M_CONV = 3, M_LAYER = 4 };
+    enum { M_LEVEL = 0, M_SUB = 1, M_ITER = 2, M_CONV = 3, M_LAYER = 4, M_DONE = 5 };
+    // The lane's flags are bits of one register, not bools: a bool that lives
+    // from trip to trip is a scalar mask, merged with three scalar
+    // instructions at every block's end.
+    //   F_WARM: the iterate began at a prediction; F_FELL: it was given up;
+    //   F_LAYERED: a layer is complete (the height output is zk, else
+    //   -999999); F_TOP: the current level's stop test
+    enum { F_WARM = 1, F_FELL = 2, F_LAYERED = 4, F_TOP = 8 };
     int mode, k, nk, left, it, nh;   // left: sub-steps of the level not yet begun
-    bool warm, fell_back, first_sub;
-    bool layered;   // a layer is complete: the height output is zk (else -999999)
+    int fl;
+    bool first_sub;   // (counts only)
     T th2, pi2, p2, t2, qv2, b2, zk, ql2, qi2, qt;
     T cape, cin, narea;
     // the previous level's pi and thv (the layer update needs both levels),
-    // and the current level's environment and stop test
+    // and the current level's environment
     T pi_prev, thv_prev;
     T e_p, e_pi, e_thv;
-    bool e_top;
     // an accessor with evaluated levels: the next one as stored (and its
     // pressure, for the LFC/EL), loaded a level ahead so that the load is in
     // flight while this level ascends
@@ -950,9 +951,8 @@ struct WarmAscent {
     // there is no history, r1 holds the caller's first guess, NaN for none)
     T r1, r2, dl1, dl2;
     // adiabat_shape at the current sub-step's start (NaN: not a pure liquid
-    // or pure ice regime), and whether the last sub-step condensed
+    // or pure ice regime, or the last sub-step did not condense)
     T gs;
-    bool sat;
     // LEVELS: the LFC/EL tracker and the previous level's pressure
     LevelTrack<T, MATH> trk;
     T pb;
@@ -962,23 +962,22 @@ struct WarmAscent {
     XC_HD __forceinline__ bool init(const Parcel<T> &pc, int nk_, T guess)
     {
         nk = nk_;
-        layered = false;
+        fl = 0;
         th2 = pc.th2; pi2 = pc.e.pi; p2 = pc.e.p; t2 = pc.t2; qv2 = pc.qv2; b2 = pc.b2;
         zk = pc.zk;
         ql2 = T(0.0); qi2 = T(0.0); qt = qv2;
         cape = T(0.0); cin = T(0.0); narea = T(0.0);
         pi_prev = pc.e.pi; thv_prev = pc.e.thv;
         k = pc.kmax;
-        e_p = pc.e.p; e_pi = pc.e.pi; e_thv = pc.e.thv; e_top = false;
+        e_p = pc.e.p; e_pi = pc.e.pi; e_thv = pc.e.thv;
         dp = T(0.0);
         left = 0; it = 0; nh = 0;
         p1 = T(0.0); t1 = T(0.0); th1 = T(0.0); qv1 = T(0.0); ql1 = T(0.0); qi1 = T(0.0);
         logp = T(0.0); thlast = T(0.0);
-        warm = false; fell_back = false; first_sub = true;
+        first_sub = true;
         x_prev = T(0.0); f_prev = T(0.0); fpr = T(0.0);
         r1 = guess; r2 = T(0.0); dl1 = T(0.0); dl2 = T(0.0);
         gs = T(NAN);
-        sat = false;
         if constexpr (LEVELS) {
             trk = LevelTrack<T, MATH>{};
             pb = pc.e.p;
@@ -997,11 +996,57 @@ struct WarmAscent {
 
     XC_HD __forceinline__ void result(ColumnOut<T> &out) const
     {
-        out.cape = cape; out.cin = cin; out.zout = layered ? zk : T(-999999.0);
+        out.cape = cape; out.cin = cin; out.zout = (fl & F_LAYERED) ? zk : T(-999999.0);
         if constexpr (LEVELS) {
             out.p_lfc = Fn<T, MATH>::div(trk.lfc, T(100.0));
             out.p_el = Fn<T, MATH>::div(trk.el, T(100.0));
         }
+    }
+
+    // One fixed-point iteration (:436-479).  HEAD: the trip's first, which may
+    // be the sub-step's first (the second never is one that began at a
+    // prediction).
+    template <bool HEAD>
+    XC_HD __forceinline__ void iterate(T fallback_tol, LaneStats &st)
+    {
+        using K = Phys<T>;
+        it = it + 1;
+        const T x = thlast;
+        fp_eval<T, MATH, ICE, PSEUDO>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, x, th2, t2, qv2,
+                                      ql2, qi2);
+        // (fast math: the products th2 and inc are not contracted into the
+        // sums after them)
+        if constexpr (MATH == MATH_FAST) xc_arrived(th2);
+        st.iterations++;
+        if (first_sub) st.first++;
+        const T d = th2 - x;
+        const T ad = d < T(0.0) ? -d : d;
+        // not converged: the reference's relaxed step; a warm-started
+        // sub-step whose first iterate missed takes the secant step instead,
+        // with the map's slope f' from the sub-steps before
+        bool again = ad > K::converge;
+        T inc = T(0.3) * d;
+        const bool head = HEAD && (fl & F_WARM) != 0 && it == 1;
+        if (HEAD) {
+            const T sec = pred_div(d, T(1.0) - fpr);
+            inc = head ? sec : inc;
+        }
+        if constexpr (MATH == MATH_FAST) xc_arrived(inc);
+        T nxt = x + inc;
+        if (HEAD) {
+            const bool miss = head && ad > fallback_tol;
+            // fallback: the reference's cold start, full iteration budget
+            nxt = miss ? th1 : nxt;
+            fl = miss ? (fl ^ F_WARM) | F_FELL : fl;
+            it = miss ? 0 : it;
+            again = again || miss;
+            st.fallbacks += miss ? 1 : 0;
+        }
+        thlast = again ? nxt : x;
+        x_prev = again ? x : x_prev;
+        f_prev = again ? th2 : f_prev;
+        // converged (:475-479): finished below, once per trip
+        mode = again ? M_ITER : M_CONV;
     }
 
     // One trip.  Returns true when the column is finished (terminated, top
@@ -1022,7 +1067,9 @@ struct WarmAscent {
         // the mask of the lanes whose mode asks for it; `mode` is made opaque
         // at the top of the trip so that the compiler cannot thread the
         // iterate-again path into an inner loop (which would make the lanes
-        // that converged wait for the slowest one again).
+        // that converged wait for the slowest one again).  Within a part every
+        // choice is a select: a branch that some lane takes in nearly every
+        // trip costs its mask's bookkeeping on top of both sides.
         xc_opaque(mode);
         st.blocks = 0;
         if (mode == M_LEVEL) {
@@ -1045,7 +1092,8 @@ struct WarmAscent {
             } else {
                 lv = level_from<T, MATH>(env_from<T, MATH>(col.raw_above(k)), e_p, pinc);
             }
-            e_p = lv.p; e_pi = lv.pi; e_thv = lv.thv; e_top = lv.top;
+            e_p = lv.p; e_pi = lv.pi; e_thv = lv.thv;
+            fl = (fl & ~F_TOP) | (lv.top ? F_TOP : 0);
             dp = lv.dp;
             left = lv.nloop;
             st.levels++;
@@ -1062,73 +1110,49 @@ struct WarmAscent {
             p2 = p2 - dp;
             pi2 = F::pow(p2 * K::rp00, K::rddcp);
             logp = log_ratio<T, MATH>(p2, p1);
+            // (fast math: the logarithm's product is not contracted into the
+            // sum below)
+            if constexpr (MATH == MATH_FAST) xc_arrived(logp);
             T g = th1;
-            if (!predict) {
-                // every sub-step cold: the flattened loop without prediction
-            } else if (nh >= 2) {
-                const T r = r1 + (r1 - r2) * pdiv(logp + dl1, dl1 + dl2);
-                g = th1 + r * logp;
-            } else if (nh == 1) {
-                g = th1 + r1 * logp;
-            } else if (r1 == r1) {
-                // the caller's guess, used once
-                g = r1;
-                r1 = T(NAN);
+            if (predict) {
+                // the history's extrapolation, or the caller's guess (used
+                // once), or none; not predict: every sub-step cold
+                const T w = pdiv(logp + dl1, dl1 + dl2);
+                const T r = nh >= 2 ? r1 + (r1 - r2) * w : r1;
+                const T gh = th1 + r * logp;
+                const T gc = r1 == r1 ? r1 : th1;
+                g = nh >= 1 ? gh : gc;
+                r1 = nh >= 1 ? r1 : T(NAN);
             }
             // a guess that is not finite or absurdly far is no guess
             const T dg = g - th1;
-            if (!((dg < T(0.0) ? -dg : dg) < T(50.0))) g = th1;
+            g = (dg < T(0.0) ? -dg : dg) < T(50.0) ? g : th1;
             thlast = g;
-            warm = g != th1;
-            fell_back = false;
+            fl = (fl & ~(F_WARM | F_FELL)) | (g != th1 ? F_WARM : 0);
             it = 0;
             st.substeps++;
             mode = M_ITER;
         }
-        // up to XC_ITERS_PER_TRIP fixed-point iterations (:436-479): most
-        // warm-started sub-steps converge at the first or second, so two per
-        // trip halve the trips that pay for the set-up blocks around them.
-        // Not unrolled: the unrolled pair, each with the evaluation's IEEE
-        // re-evaluation path, no longer fits the 64 registers
-#pragma unroll 1
-        for (int rep = 0; rep < XC_ITERS_PER_TRIP; ++rep) {
-            if (mode != M_ITER) continue;
-            st.blocks |= 4u << rep;
-            it = it + 1;
-            const T x = thlast;
-            fp_eval<T, MATH, ICE, PSEUDO>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, x, th2, t2,
-                                          qv2, ql2, qi2);
-            st.iterations++;
-            if (first_sub) st.first++;
-            const T d = th2 - x;
-            const T ad = d < T(0.0) ? -d : d;
-            if (it > 100) {
+        // two iterations per trip: most warm-started sub-steps converge at the
+        // first or second, so the pair halves the trips that pay for the
+        // set-up blocks around them
+        if (mode == M_ITER) {
+            st.blocks |= 4u;
+            iterate<true>(fallback_tol, st);
+        }
+        if (mode == M_ITER) {
+            st.blocks |= 8u;
+            iterate<false>(fallback_tol, st);
+        }
+        if (it > 100) {
+            // (once over, whatever the evaluation gave, :464)
+            if (mode == M_ITER || mode == M_CONV) {
                 st.nonconverged++;
                 cape = T(0.0);
                 cin = T(0.0);
                 // a column stopped by the iteration limit reports no levels
                 if constexpr (LEVELS) trk = LevelTrack<T, MATH>{};
-                return true;
-            }
-            if (warm && it == 1 && ad > fallback_tol) {
-                // fallback: the reference's cold start, full iteration budget
-                thlast = th1;
-                warm = false;
-                fell_back = true;
-                it = 0;
-                st.fallbacks++;
-            } else if (ad > K::converge) {
-                // the reference's relaxed step; a warm-started sub-step whose
-                // first iterate missed takes the secant step instead, with the
-                // map's slope f' from the sub-steps before
-                T nxt = x + T(0.3) * (th2 - x);
-                if (warm && it == 1) nxt = x + pdiv(th2 - x, T(1.0) - fpr);
-                thlast = nxt;
-                x_prev = x;
-                f_prev = th2;
-            } else {
-                // converged (:475-479): finished below, once per trip
-                mode = M_CONV;
+                mode = M_DONE;
             }
         }
         if (mode == M_CONV) {
@@ -1136,17 +1160,12 @@ struct WarmAscent {
             // the iterate that converged.  The slope f' of the map from this
             // sub-step's last two iterates (kept from an earlier sub-step
             // when it converged at its first)
+            st.blocks |= 16u;
             const T x = thlast;
-            if (it >= 2) {
-                const T dx = x - x_prev;
-                if (dx != T(0.0)) {
-                    const T sl = pdiv(th2 - f_prev, dx);
-                    fpr = sl < T(-10.0) ? T(-10.0) : (sl > T(0.9) ? T(0.9) : sl);
-                }
-            }
-        }
-        if (mode == M_CONV) st.blocks |= 16u;
-        if (mode == M_CONV && warm) {
+            const T dx = x - x_prev;
+            T sl = pdiv(th2 - f_prev, dx);
+            sl = sl < T(-10.0) ? T(-10.0) : (sl > T(0.9) ? T(0.9) : sl);
+            fpr = it >= 2 && dx != T(0.0) ? sl : fpr;
             // Would the reference's own solve, from the cold start th1 with
             // its relaxed step (contraction c = 1 - 0.3 (1 - f') per
             // iteration), take more than about 50 iterations here?  Then it
@@ -1158,11 +1177,10 @@ struct WarmAscent {
             const T c = T(1.0) - T(0.3) * (T(1.0) - fpr);
             const T c2 = c * c, c4 = c2 * c2, c8 = c4 * c4, c16 = c8 * c8;
             const T c50 = c16 * c16 * c16 * c2;
-            const T e0 = thlast - th1;
-            if ((e0 < T(0.0) ? -e0 : e0) * c50 > K::converge) {
+            const T e0 = x - th1;
+            if ((fl & F_WARM) != 0 && (e0 < T(0.0) ? -e0 : e0) * c50 > K::converge) {
                 thlast = th1;
-                warm = false;
-                fell_back = true;
+                fl = (fl & ~F_WARM) | F_FELL;
                 it = 0;
                 st.fallbacks++;
                 mode = M_ITER;
@@ -1176,38 +1194,29 @@ struct WarmAscent {
             // where the condensate is all liquid (above 0 degC; everywhere
             // for the liquid adiabat) or all ice (below -40 degC); none in
             // the ice adiabat's mixed range
-            const bool sat_now = qv2 < qt;
             T ge = T(NAN);
             if (PSEUDO && predict) {
                 const bool ice = ICE && t2 < T(233.15);
-                if (ice || !ICE || t2 > T(273.15)) ge = adiabat_shape<T>(t2, p2, th2, ice);
+                const T shape = adiabat_shape<T>(t2, p2, th2, ice);
+                ge = qv2 < qt && (ice || !ICE || t2 > T(273.15)) ? shape : T(NAN);
             }
-            if (logp != T(0.0)) {
-                const T xs = x + pdiv(th2 - x, T(1.0) - fpr);
-                const T rn = pdiv(xs - th1, logp);
-                // saturated ascent within one phase: a history whose
-                // second-order extrapolation is this rate scaled by the
-                // shape's change between the sub-steps' midpoints (log-linear
-                // in ln p, linearised):
-                // r = rn (1 + (ge / gs - 1) (logp' + dl1) / (2 dl1)).
-                // Otherwise the measured history; a second-order guess that
-                // failed marks a change of regime (saturation, ice onset):
-                // the older rate belongs to the other side, so restart at
-                // first order
-                const bool shaped = sat && sat_now && gs == gs && ge == ge;
-                const T r2n = shaped ? rn * (T(2.0) - pdiv(ge, gs)) : r1;
-                const T dl2n = shaped ? logp : dl1;
-                nh = shaped ? 2 : (fell_back && nh >= 2 ? 1 : (nh < 2 ? nh + 1 : 2));
-                r2 = r2n;
-                dl2 = dl2n;
-                r1 = rn;
-                dl1 = logp;
-            } else {
-                nh = 0;
-                r1 = T(NAN);
-            }
+            const T xs = x + pdiv(th2 - x, T(1.0) - fpr);
+            const T rn = pdiv(xs - th1, logp);
+            // saturated ascent within one phase: a history whose second-order
+            // extrapolation is this rate scaled by the shape's change between
+            // the sub-steps' midpoints (log-linear in ln p, linearised):
+            // r = rn (1 + (ge / gs - 1) (logp' + dl1) / (2 dl1)).  Otherwise
+            // the measured history; a second-order guess that failed marks a
+            // change of regime (saturation, ice onset): the older rate belongs
+            // to the other side, so restart at first order
+            const bool shaped = gs == gs && ge == ge;
+            r2 = shaped ? rn * (T(2.0) - pdiv(ge, gs)) : r1;
+            dl2 = shaped ? logp : dl1;
+            const int nm = (fl & F_FELL) != 0 && nh >= 2 ? 1 : (nh < 2 ? nh + 1 : 2);
+            nh = logp != T(0.0) ? (shaped ? 2 : nm) : 0;
+            r1 = logp != T(0.0) ? rn : T(NAN);
+            dl1 = logp;
             gs = ge;
-            sat = sat_now;
             if (PSEUDO) {
                 qt = qv2;
                 ql2 = T(0.0);
@@ -1227,12 +1236,12 @@ struct WarmAscent {
                 layer_update<T, MATH>(th2, qv2, ql2, qi2, e_thv, e_pi, e_p, thv_prev, pi_prev,
                                       b1, b2, dz, cape, cin, narea);
             zk = zk + dz;
-            layered = true;
             pi_prev = e_pi; thv_prev = e_thv;
-            if ((e_top && b2 < T(0.0)) || !(k < nk - 1)) return true;
-            mode = M_LEVEL;
+            const bool stop = ((fl & F_TOP) != 0 && b2 < T(0.0)) || !(k < nk - 1);
+            fl = fl | F_LAYERED;
+            mode = stop ? M_DONE : M_LEVEL;
         }
-        return false;
+        return mode == M_DONE;
     }
 };
 
