@@ -442,11 +442,13 @@ __host__ __device__ __forceinline__ uint32_t work_parts(uint32_t grid)
 
 // PREDICT: the warm start (false: the same loop with every sub-step cold).
 // LEVELS: also the LFC and EL.
-// Held to 72 VGPRs, 7 waves per SIMD: the ascent is bound by VALU issue (4
-// waves per SIMD are within 6 % of 8), and at 64 VGPRs the compiler spilled
-// scalar registers to VGPR lanes and shuffled more (7 waves ran 1.5 % faster).
+// Held to 80 VGPRs, 6 waves per SIMD: the ascent is bound by VALU issue, which
+// 4 waves already fill, and the fewer waves a grid has, the fewer of its lanes
+// wait at the end for the last columns.  2^21 columns of 137 levels,
+// pseudo-ice: 7.60 ms with 6 waves, 7.95 with 7, 7.92 with 8, 7.67 with 5;
+// 524 288 of 37 with levels: 1.41, 1.45, 1.50, 1.50.
 template <bool ICE, bool PSEUDO, bool PREDICT, bool STATS, bool LEVELS = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 6)))
 warm_ascent_kernel(CapeGridArgs a, int cpw)
 {
     using T = float;
