@@ -189,3 +189,50 @@ def test_ragged_full_size(hip, oracle_lib):
                             d['ts'][idx], d['tds'][idx], pinc=500., source=int(key[1]),
                             ml_depth=500., adiabat=int(key[2]))
         assert cape_ok(plain[0][idx], o[0]).all() and cape_ok(plain[1][idx], o[1]).all()
+
+
+@pytest.mark.parametrize('warm', [False, True])
+@pytest.mark.parametrize('ncol', [1, 63, 65, 700])
+def test_staging_tile_edges(hip, ncol, warm):
+    """Level counts at the edges of the staging tiles (64 columns by 64
+    levels), in columns that share tiles: a column's values are those of a
+    grid call on it, bit for bit (the same functions on the same values)."""
+    import torch
+
+    from xcape_amd.ragged import RaggedBatch, RaggedPlan
+    rng = np.random.default_rng(ncol)
+    heights = np.asarray([6, 63, 64, 65, 127, 128, 129])
+    nlev = rng.choice(heights, ncol)
+    off = np.zeros(ncol + 1, np.int64)
+    off[1:] = np.cumsum(nlev)
+    lev = {k: np.empty(off[-1], np.float32) for k in ('p', 't', 'td')}
+    sfc = {k: np.empty(ncol, np.float32) for k in ('ps', 'ts', 'tds')}
+    groups = [(nk, np.nonzero(nlev == nk)[0]) for nk in heights]
+    for nk, idx in groups:
+        if not len(idx):
+            continue
+        c = synthetic.sigma_columns(len(idx), int(nk), int(nk))
+        rows = off[idx][:, None] + np.arange(nk)[None, :]
+        for k in lev:
+            lev[k][rows] = c[k]
+        for k in sfc:
+            sfc[k][idx] = c[k]
+    src = np.full(ncol, 2, np.int32)
+    adi = rng.choice(np.asarray([1, 3], np.int32), ncol)
+    b = RaggedBatch(off, lev['p'], lev['t'], lev['td'], sfc['ps'], sfc['ts'], sfc['tds'], src, adi)
+    plan = RaggedPlan(b, pinc=500., ml_depth=500., chunk=64, tile=16, cols=64, warm_start=warm)
+    plan.run()
+    torch.cuda.synchronize()
+    got = [x.cpu().numpy() for x in (b.cape, b.cin, b.mulev, b.zmulev)]
+    plan.close()
+    for nk, idx in groups:
+        rows = off[idx][:, None] + np.arange(nk)[None, :]
+        for ad in (1, 3):
+            m = adi[idx] == ad
+            if not m.any():
+                continue
+            args = [lev[k][rows[m]] for k in ('p', 't', 'td')]
+            args += [sfc[k][idx[m]] for k in ('ps', 'ts', 'tds')]
+            ref = hip.cape(*args, pinc=500., source=2, adiabat=ad, warm_start=warm)
+            for g, r in zip(got, ref):
+                np.testing.assert_array_equal(g[idx[m]], r)
