@@ -692,9 +692,9 @@ hipError_t launch_cape(const CapeGridArgs &a, int block, hipStream_t s)
 // and shares the columns out: a wave runs a block of the trip whenever one of
 // its columns is there, so fewer columns are fewer blocks, and the lanes
 // without a column repeat one (a wave with few active lanes runs slower than a
-// full one).  121 x 97 columns of 50 levels, pseudo-ice: 1030 us 64 to a wave,
-// 922 with 12; 1024 columns: 982 us and 698 with one; more waves than SIMDs are
-// slower again (65 536 columns of 137 levels: 859 us, 988 with 32).  The
+// full one).  121 x 97 columns of 50 levels, pseudo-ice: 713 us 64 to a wave,
+// 621 with 12; 1024 columns: 694 us and 448 with one; more waves than SIMDs are
+// slower again (65 536 columns of 137 levels: 516 us, 647 with 32).  The
 // counted launches take 64, so that no column is counted twice.
 template <bool ICE, bool PSEUDO, bool PREDICT, bool STATS, bool LEVELS>
 int ascent_grid(int block, int64_t ncol, int *cpw)
@@ -722,8 +722,8 @@ int ascent_grid(int block, int64_t ncol, int *cpw)
     int64_t g = (ncol + cols - 1) / cols;
     // a multiple of the work parts, so that every part has as many waves:
     // rounded up, since one column too many for a part's waves is a second
-    // ascent for one of them (121 x 97 columns: 1526 us with 40 blocks, 1030
-    // with 48)
+    // ascent for one of them (121 x 97 columns: 961 us with 40 blocks, 713
+    // with 48, 64 columns to a wave)
     if (g > (int64_t)WORK_PARTS) g = (g + WORK_PARTS - 1) / WORK_PARTS * WORK_PARTS;
     const int64_t full = cus * per_cu[slot];
     if (g > full) g = full >= (int64_t)WORK_PARTS ? full - full % WORK_PARTS : full;
