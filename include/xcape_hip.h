@@ -18,7 +18,7 @@
  * calls are synchronous; with stream NULL they run on a stream of the calling
  * thread's own.  Some calls also queue work on a second stream of the calling
  * thread (the helicity launches of the combined call, and the staging copies
- * of a warm-started or helicity-only grid of many column-contiguous columns),
+ * of a warm-started grid of many column-contiguous columns),
  * forked after the work already queued on `stream` and joined back into
  * `stream` before the call returns, so a call stays ordered as one unit.
  */
@@ -104,9 +104,9 @@ const char *xcape_last_error(void);
 int xcape_device_count(void);
 
 /*
- * Host-array calls (no XCAPE_DEVICE_PTRS, column-contiguous arrays) stream
- * their columns in chunks of about 128 MB of input (XCAPE_HOST_CHUNK_MB)
- * through pinned host memory and device buffers that stay allocated for the
+ * Host-array calls (no XCAPE_DEVICE_PTRS, column-contiguous arrays, double
+ * ones included) stream their columns in chunks of about 128 MB of input
+ * (XCAPE_HOST_CHUNK_MB; up to 64 MB go as one chunk) through pinned host memory and device buffers that stay allocated for the
  * next call: at most two such staging sets per process (three slots of
  * pinned input, pinned output and device buffers each), so at most two
  * host-array calls stream at once and a third waits for one of them.  This
@@ -228,9 +228,8 @@ int xcape_cape_levels_f64(const float *p, int p_shared, const int32_t *start_lev
  * m/s; with XCAPE_INPUT_F64 the ten input pointers point at double arrays.
  * Outputs: srh_rm, srh_lm (ncol,) FP64; rm, lm, mean6 (ncol, 2) as
  * (u, v) pairs (the reference's (2, n2) Fortran arrays), all three NULL to
- * skip them.  Grids of 2^18 column-contiguous columns or more are staged in
- * four parts, each part's launch on a second stream of the calling thread
- * while the next part is copied (joined back as above).
+ * skip them.  The profiles are read where they lie, in either layout: device
+ * calls take no scratch.
  */
 int xcape_srh_f32(const float *p, int p_shared, const int32_t *start_lev,
                   const float *t, const float *td, const float *u, const float *v,
@@ -252,11 +251,12 @@ int xcape_srh_f64(const float *p, int p_shared, const int32_t *start_lev,
 
 /*
  * CAPE/CIN (as xcape_cape_f32) and the helicity chain (as xcape_srh_f32) of
- * the same columns in one call: column-contiguous profiles are staged
- * level-major once for both, and the helicity launch runs on a second stream
+ * the same columns in one call: the helicity launch runs on a second stream
  * beside the ascent (forked after the work queued on `stream`, with the warm
- * start after the setup pass, with the copies of the winds; joined back
- * before the call returns or anything later on `stream` runs).  No single
+ * start after the setup pass; joined back before the call returns or anything
+ * later on `stream` runs).  From 2^20 warm-started column-contiguous columns
+ * on, it reads the CAPE launches' level-major copies, and copies of the winds
+ * made beside the ascent.  No single
  * reference counterpart: it serves callers that need both calls above.
  */
 int xcape_cape_srh_f32(const float *p, int p_shared, const int32_t *start_lev,
