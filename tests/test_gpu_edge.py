@@ -153,3 +153,17 @@ def test_ragged_plans(hip, ref, adiabat, warm):
         plan.close()
         _check(f'ragged warm={warm} s{src} ml{ml} a{adiabat}', got, st['nonconverged'],
                ref[(src, ml, adiabat)])
+
+
+@pytest.mark.parametrize('adiabat', ADIABATS)
+def test_evaluations_counted_up_to_the_limit(hip, adiabat):
+    """The warm start's loop without predictions does the plain method's
+    evaluations, one by one, those of the columns that exceed the limit
+    included: the same counts."""
+    arr = edge_cases.grid()
+    for src, ml in edge_cases.CASES:
+        kw = dict(pinc=500., source=src, ml_depth=ml, adiabat=adiabat, stats=True)
+        plain = hip.cape(*arr, **kw)[4]
+        cold = hip.cape(*arr, warm_start='cold', **kw)[4]
+        for k in ('levels', 'substeps', 'iterations', 'nonconverged'):
+            assert cold[k] == plain[k], (src, ml, k)

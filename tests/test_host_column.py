@@ -165,3 +165,21 @@ def test_edge_branches(host_lib, adiabat):
         assert cape_ok(warm[0][ok], ref[0][ok]).all() and cape_ok(warm[1][ok], ref[1][ok]).all()
         stopped = (ref[0] == 0) & (ref[1] == 0)
         assert np.all(warm[0][stopped] == 0) and np.all(warm[1][stopped] == 0)
+
+
+@pytest.mark.parametrize('adiabat', [1, 2, 3, 4])
+def test_iterations_of_stopped_columns(host_lib, adiabat):
+    """A solve that exceeds the limit ends at its 101st evaluation, in the
+    warm start's loop (two evaluations to a trip) as in the reference's.  Mixed
+    parcels lifted from 300 to 600 hPa, some of which stop at their first
+    sub-step: without a surrogate it starts cold, so both methods count the
+    same evaluations of it."""
+    n = 2000
+    c = S.sigma_columns(n, 30, 6)
+    p, t, td, ts, tds = (c[k].copy() for k in ('p', 't', 'td', 'ts', 'tds'))
+    ps = np.linspace(300, 600, n).astype(np.float32)
+    p = np.minimum(p, ps[:, None] - 10)
+    _, sp = host_cape(host_lib, p, t, td, ps, ts, tds, 3, adiabat, False)
+    _, sw = host_cape(host_lib, p, t, td, ps, ts, tds, 3, adiabat, True)
+    assert sw['nonconverged'] > 0
+    assert sw['first'] == sp['first']

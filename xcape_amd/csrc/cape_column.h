@@ -1148,6 +1148,13 @@ struct WarmAscent {
             // (once over, whatever the evaluation gave, :464)
             if (mode == M_ITER || mode == M_CONV) {
                 st.nonconverged++;
+                // the limit falls on the trip's first evaluation for a sub-step
+                // that began with one: the second is over it, and not counted
+                if (it > 101) {
+                    st.iterations--;
+                    if (first_sub) st.first--;
+                    st.blocks &= ~8u;
+                }
                 cape = T(0.0);
                 cin = T(0.0);
                 // a column stopped by the iteration limit reports no levels
