@@ -646,3 +646,21 @@ def test_small_launches_match_the_large_loop(hip, adiabat, ncol, nk):
     for a, b in zip(small, large[:4]):
         assert torch.equal(a, b)
     assert large[4]['columns'] == ncol
+
+
+@pytest.mark.parametrize('adiabat', [1, 2, 3, 4])
+@pytest.mark.parametrize('mode', [dict(fast_math=True), dict(fp64=True)])
+@pytest.mark.parametrize('ncol', [1, 1025, 4096, 4097, 20011, 131072])
+def test_small_launches_match_the_large_in_fast_math_and_fp64(hip, mode, adiabat, ncol):
+    """Fast math and FP64 spread a small launch's columns over the waves too,
+    in a kernel of their own (fast reversible-liquid launches of up to 4 columns
+    a wave, the others of up to 64): on both sides of these limits a column's
+    result is that of a launch larger than all of them, bit for bit."""
+    import torch
+    c = synthetic.sigma_columns_torch(131073, 16, 40 + adiabat)
+    args = [c[k] for k in ('p', 't', 'td', 'ps', 'ts', 'tds')]
+    kw = dict(pinc=2500., source=1 + adiabat % 3, adiabat=adiabat, **mode)
+    whole = hip.cape(*args, **kw)
+    part = hip.cape(*(a[:ncol].contiguous() for a in args), **kw)
+    for w, p in zip(whole, part):
+        assert torch.equal(p, w[:ncol])

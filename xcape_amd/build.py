@@ -33,7 +33,10 @@ UNITS = {
     'capi.hip': ['-ffp-contract=off'],
     # MFMA operands and accumulators in VGPRs (not AGPRs): the surrogate's
     # evaluation shares the ascent kernel's register budget
-    'cape_accurate.hip': ['-ffp-contract=off', '-mllvm', '-amdgpu-mfma-vgpr-form=1'],
+    # (loops at 64-byte boundaries: where one falls moves a launch of few waves
+    # by up to 6 %; 110 000 columns, reversible-liquid, 982 us against 1042 without)
+    'cape_accurate.hip': ['-ffp-contract=off', '-mllvm', '-amdgpu-mfma-vgpr-form=1',
+                          '-falign-loops=64'],
     'cape_fast.hip': ['-ffp-contract=fast-honor-pragmas', '-mllvm', '-amdgpu-mfma-vgpr-form=1'],
     'ragged.hip': ['-ffp-contract=off'],
     'mlp.hip': ['-ffp-contract=fast'],

@@ -620,7 +620,14 @@ hipError_t launch_srh(const CapeGridArgs &a, dim3 grid, int block, hipStream_t s
 // pseudo-liquid, take 477 us one to a wave and 574 us 64 to a wave; 65 536 of
 // 137 levels, pseudo-ice, 1.41 ms with the small launches' loop and 1.71
 // without; 131 072, 2.24 and 2.28; 262 144, 4.00 and 3.81.
-inline int few_columns(int64_t ncol)
+//
+// FP64 and fast math have no loop of their own for few waves and gain by the
+// spreading alone: 2000 columns of 40 levels 1.05 to 1.2 times, 64 000 not any
+// more.  The fast reversible-liquid kernel is spread up to four columns to a
+// wave only: 2000 columns 501 us against 522 without, 20 000 549 against 535,
+// 110 000 759 against 725 (the loop's instructions are the same; aligned to 64
+// bytes, it is as fast at 110 000, and the pseudo-liquid one 3 % slower).
+inline int few_columns(int64_t ncol, bool fast_reversible_liquid)
 {
     static const int simds = [] {
         int dev = 0, ncu = 0;
@@ -628,7 +635,7 @@ inline int few_columns(int64_t ncol)
         (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
         return 4 * (ncu > 0 ? ncu : 256);
     }();
-    if (ncol > (int64_t)2 * 64 * simds) return 0;
+    if (ncol > (int64_t)(fast_reversible_liquid ? 4 : 2 * 64) * simds) return 0;
     const int64_t c = (ncol + simds - 1) / simds;
     return c < 64 ? (int)c : 64;
 }
@@ -662,7 +669,8 @@ hipError_t launch_cape_f(const CapeGridArgs &a, int block, hipStream_t s)
 {
     // the counted launches keep the large grids' loop
     if constexpr (!STATS) {
-        if (const int cpw = few_columns(a.ncol))
+        const bool frl = XC_MATH == MATH_FAST && a.adiabat == 2;
+        if (const int cpw = few_columns(a.ncol, frl))
             return launch_cape_s<T, IDX, STATS, LEVELS, true>(a, block, cpw, s);
     }
     return launch_cape_s<T, IDX, STATS, LEVELS, false>(a, block, 0, s);
