@@ -664,3 +664,27 @@ def test_small_launches_match_the_large_in_fast_math_and_fp64(hip, mode, adiabat
     part = hip.cape(*(a[:ncol].contiguous() for a in args), **kw)
     for w, p in zip(whole, part):
         assert torch.equal(p, w[:ncol])
+
+
+@pytest.mark.parametrize('adiabat', [1, 2, 3, 4])
+@pytest.mark.parametrize('ncol', [1, 63, 2111, 131072])
+def test_three_loops_agree(hip, ncol, adiabat):
+    """The accurate mode's loops: a launch of more than two waves per SIMD
+    leaves lanes and phases out, a counted one below that leaves out lanes, an
+    uncounted one nothing.  A column's result is the same in each, bit for
+    bit, columns that stop at the iteration limit and NaN levels included."""
+    import edge_cases
+    import torch
+    c = synthetic.sigma_columns_torch(131073, 30, 90 + adiabat)
+    args = [c[k] for k in ('p', 't', 'td', 'ps', 'ts', 'tds')]
+    for a, e in zip(args, edge_cases.grid()):
+        a[:128] = torch.from_numpy(e).cuda()
+    kw = dict(pinc=500., source=1 + adiabat % 3, adiabat=adiabat)
+    whole = hip.cape(*args, **kw)
+    part = [a[:ncol].contiguous() for a in args]
+    few = hip.cape(*part, **kw)
+    counted = hip.cape(*part, stats=True, **kw)
+    for w, f, m in zip(whole, few, counted):
+        w = w[:ncol].nan_to_num(nan=-7e7)
+        assert torch.equal(f.nan_to_num(nan=-7e7), w)
+        assert torch.equal(m.nan_to_num(nan=-7e7), w)

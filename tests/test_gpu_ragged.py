@@ -236,3 +236,40 @@ def test_staging_tile_edges(hip, ncol, warm):
             ref = hip.cape(*args, pinc=500., source=2, adiabat=ad, warm_start=warm)
             for g, r in zip(got, ref):
                 np.testing.assert_array_equal(g[idx[m]], r)
+
+
+@pytest.mark.parametrize('cols', [16, 64, 256])
+@pytest.mark.parametrize('ncol', [1, 65, 1000, 33000])
+def test_small_plain_batches_match_the_large(hip, ncol, cols):
+    """A plain batch of at most two waves per SIMD iterates with the few-wave
+    loop, a larger one with the large grids': a column's result and its counts
+    do not depend on the batch it is in, bit for bit.  (33 000 columns are few
+    at 64 to a wave, many at 16.)"""
+    import torch
+
+    from xcape_amd.ragged import RaggedBatch, RaggedPlan
+    d = synthetic.ragged_columns(140000, 8)
+    rng = np.random.default_rng(ncol)
+    adi = rng.integers(1, 5, 140000).astype(np.int32)
+
+    def run(n, stats):
+        off = d['offsets'][:n + 1]
+        lev = [d[k][:off[-1]] for k in ('p', 't', 'td')]
+        sfc = [d[k][:n] for k in ('ps', 'ts', 'tds')]
+        b = RaggedBatch(off, *lev, *sfc, d['source'][:n], adi[:n])
+        plan = RaggedPlan(b, pinc=2500., ml_depth=500., chunk=64, tile=16, cols=cols)
+        plan.run()
+        torch.cuda.synchronize()
+        out = [x.cpu().numpy() for x in (b.cape, b.cin, b.mulev, b.zmulev)]
+        st = plan.run(stats=True) if stats else None
+        torch.cuda.synchronize()
+        again = [x.cpu().numpy() for x in (b.cape, b.cin, b.mulev, b.zmulev)]
+        plan.close()
+        for x, y in zip(out, again):
+            np.testing.assert_array_equal(x, y)
+        return out, st
+    whole, _ = run(140000, False)
+    part, st = run(ncol, True)
+    for w, p in zip(whole, part):
+        np.testing.assert_array_equal(p, w[:ncol])
+    assert st['columns'] == np.count_nonzero(d['ts'][:ncol] > 0)

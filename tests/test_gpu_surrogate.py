@@ -284,3 +284,31 @@ def test_committed_surrogate_gain_full_size(torch):
                                                               (ce[off], ke[off])])
         assert ill.all() and matched.all(), (off, ill, matched)
     np.testing.assert_array_equal(out_s[2].cpu().numpy(), out_e[2].cpu().numpy())
+
+
+@pytest.mark.parametrize('adiabat', [1, 2, 3, 4])
+@pytest.mark.parametrize('ncol', [1, 777])
+def test_small_logging_launch_matches_the_large(torch, ncol, adiabat):
+    """The training data's logger iterates with the few-wave loop up to two
+    waves per SIMD: its records of the first columns are among those of a
+    larger launch, bit for bit, as many as the columns' sub-steps kept."""
+    from xcape_amd import _hip, surrogate, synthetic
+    c = synthetic.sigma_columns_torch(131073, 12, 60 + adiabat)
+    names = ('p', 't', 'td', 'ps', 'ts', 'tds')
+    P = _hip._ptr
+
+    def log(n):
+        cap = n * 120
+        out = torch.empty((cap, 5), dtype=torch.float32, device='cuda')
+        count = torch.zeros(1, dtype=torch.int64, device='cuda')
+        a = [c[k][:n].contiguous() for k in names]
+        _hip.check(_hip.lib().xcape_surrogate_log_f32(
+            *(P(x) for x in a), 12, n, 1000., 2, 500., adiabat, 0.5, 3, 0, P(out), cap, P(count),
+            surrogate._stream()))
+        got = int(count.item())
+        assert got <= cap
+        return out[:got].cpu().numpy()
+    large, small = log(131073), log(ncol)
+    assert len(small) > 0
+    kept = set(map(bytes, np.ascontiguousarray(large)))
+    assert all(bytes(r) in kept for r in np.ascontiguousarray(small))

@@ -36,6 +36,9 @@ namespace xcape {
 
 enum { SRC_SURFACE = 1, SRC_MU = 2, SRC_ML = 3 };
 
+// The accurate mode's loops on the device (solve_raw).
+enum { LOOP_LARGE = 0, LOOP_MASKS = 1, LOOP_FEW = 2 };
+
 // Makes v's value unknown to the optimiser at this point (no code).
 XC_HD __forceinline__ void xc_opaque(int &v)
 {
@@ -333,26 +336,31 @@ XC_HD __forceinline__ bool solve_substep_ops(T p2, T pi2, T logp, T t1, T th1, T
 // gives, :464); `ok`: every evaluation was in the raw kernels' range, and in
 // the regime.
 //
-// FEW = false, for launches that fill the device: a lane that has converged
+// LOOP_LARGE, for launches that fill the device: a lane that has converged
 // leaves the loop, and an ice adiabat's wave leaves out, in each evaluation,
 // the phase none of its lanes still iterating has (its lanes climb their
 // columns together: most evaluations are above 0 degC or below -40 degC on
 // every lane.  2^20 columns of 137 levels, pseudo-ice: 16.9 ms without, 12.2
 // with the regimes).
 //
-// FEW = true, for launches of a wave or so per SIMD, which wait for every
+// LOOP_MASKS: the same without the regimes, whose votes a wave that has its
+// SIMD to itself waits for (1000 columns of 40 levels, pseudo-ice, counted:
+// 1250 us with them, 1035 without).
+//
+// LOOP_FEW, for launches of a wave or so per SIMD, which wait for every
 // instruction: a lane that has converged keeps its iterate, so the evaluations
 // it goes on taking part in give its result again, and an iteration costs one
 // compare, one select and one branch beside the evaluation, with no execution
 // masks.  The regime is the caller's (REGIME), once for the whole sub-step.
 // (4096 columns of 40 levels, pseudo-liquid: 652 us with masks, 573 without;
 // 524 288 columns of 37 levels: 3.08 ms with, 3.40 without.)
-template <bool ICE, bool PSEUDO, bool FEW, int REGIME>
+template <bool ICE, bool PSEUDO, int LOOP, int REGIME>
 __device__ __forceinline__ void solve_raw(float p2, float pi2, float logp, float t1, float th1,
                                           float qv1, float ql1, float qi1, float qt, float &th2,
                                           float &t2, float &qv2, float &ql2, float &qi2,
                                           bool &more, bool &ok, LaneStats &st)
 {
+    constexpr bool FEW = LOOP == LOOP_FEW;
     // running maximum (minimum) by the median with an infinity the optimiser
     // does not know (one instruction, no canonicalisation)
     float inf = INFINITY;
@@ -364,7 +372,7 @@ __device__ __forceinline__ void solve_raw(float p2, float pi2, float logp, float
     fp_eval_raw<ICE, PSEUDO, R>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, x, th2, t2, qv2, ql2, \
                                 qi2, arg)
     for (;;) {
-        if constexpr (ICE && !FEW) {
+        if constexpr (ICE && LOOP == LOOP_LARGE) {
             const float tx = x * pi2;
             if (__builtin_amdgcn_ballot_w64(!regime_hot(p2, tx)) == 0) XC_EVAL(REG_LIQUID);
             else if (__builtin_amdgcn_ballot_w64(!regime_cold(p2, tx)) == 0) XC_EVAL(REG_ICE);
@@ -412,7 +420,7 @@ __device__ __forceinline__ void solve_raw(float p2, float pi2, float logp, float
 // rise with the latent heat), and checked after the loop.  A sub-step that
 // left the raw kernels' range is solved again from its start with the
 // library's operations, whose iterates up to there are the same.
-template <typename T, int MATH, bool ICE, bool PSEUDO, bool FEW>
+template <typename T, int MATH, bool ICE, bool PSEUDO, int LOOP>
 XC_HD __forceinline__ bool solve_substep(T p1, T p2, T pi2, T t1, T th1, T qv1, T ql1, T qi1,
                                          T qt, T &th2, T &t2, T &qv2, T &ql2, T &qi2,
                                          LaneStats &st)
@@ -423,23 +431,23 @@ XC_HD __forceinline__ bool solve_substep(T p1, T p2, T pi2, T t1, T th1, T qv1, 
         bool more = false, ok = false;
         const uint32_t it0 = st.iterations;
         bool done = false;   // wave-uniform
-        if constexpr (ICE && FEW) {
+        if constexpr (ICE && LOOP == LOOP_FEW) {
             const float tx = th1 * pi2;
             if (__builtin_amdgcn_ballot_w64(!regime_hot(p2, tx - 0.1f)) == 0) {
-                solve_raw<ICE, PSEUDO, true, REG_LIQUID>(p2, pi2, logp, t1, th1, qv1, ql1, qi1,
+                solve_raw<ICE, PSEUDO, LOOP, REG_LIQUID>(p2, pi2, logp, t1, th1, qv1, ql1, qi1,
                                                          qt, th2, t2, qv2, ql2, qi2, more, ok,
                                                          st);
                 done = __builtin_amdgcn_ballot_w64(!ok) == 0;
             } else if (__builtin_amdgcn_ballot_w64(!regime_cold(p2, tx + 3.0f)) == 0) {
-                solve_raw<ICE, PSEUDO, true, REG_ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt,
+                solve_raw<ICE, PSEUDO, LOOP, REG_ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt,
                                                       th2, t2, qv2, ql2, qi2, more, ok, st);
                 done = __builtin_amdgcn_ballot_w64(!ok) == 0;
             }
         }
         if (!done) {
             st.iterations = it0;
-            solve_raw<ICE, PSEUDO, FEW, REG_MIXED>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, th2,
-                                                   t2, qv2, ql2, qi2, more, ok, st);
+            solve_raw<ICE, PSEUDO, LOOP, REG_MIXED>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, th2,
+                                                    t2, qv2, ql2, qi2, more, ok, st);
             if (__builtin_expect(!ok, 0)) {
                 st.iterations = it0;
                 return solve_substep_ops<T, MATH_LIB, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1,
@@ -765,9 +773,9 @@ struct NoLog {
 };
 
 // Reference driver: nested loops, cold start.  LEVELS: also the LFC and EL
-// (LevelTrack).  FEW: solve_raw's loop for launches of few waves.
+// (LevelTrack).  LOOP: solve_raw's loop.
 template <typename T, int MATH, bool ICE, bool PSEUDO, class C, class LOG = NoLog,
-          bool LEVELS = false, bool FEW = false>
+          bool LEVELS = false, int LOOP = LOOP_LARGE>
 XC_HD void cape_column(const C &col, int nk, T pinc, int source, T ml_depth,
                        ColumnOut<T> &out, LaneStats &st, const LOG &log = LOG())
 {
@@ -807,7 +815,7 @@ XC_HD void cape_column(const C &col, int nk, T pinc, int source, T ml_depth,
             pi2 = Fn<T, MATH>::pow(p2 * K::rp00, K::rddcp);
             st.substeps++;
             const uint32_t it0 = st.iterations;
-            const bool ok = solve_substep<T, MATH, ICE, PSEUDO, FEW>(
+            const bool ok = solve_substep<T, MATH, ICE, PSEUDO, LOOP>(
                 p1, p2, pi2, t1, th1, qv1, ql1, qi1, qt, th2, t2, qv2, ql2, qi2, st);
             if (first_sub) st.first += st.iterations - it0;
             first_sub = false;

@@ -185,18 +185,18 @@ namespace XC_NS {
 // column per lane.  STATS: accumulate the work counters into a.stats (a
 // separate instantiation, so that the counters do not occupy registers in
 // the timed kernels).  LEVELS: also the LFC and EL (a.p_lfc, a.p_el).
-// FEW (small launches, see few_columns): `cpw` columns to a wave, the lanes
-// beyond them on its columns again.  (Waves with few lanes switched on run
+// LOOP: solve_raw's; LOOP_FEW (small launches, see few_columns) also puts `cpw`
+// columns to a wave, the lanes beyond them on its columns again.  (Waves with few lanes switched on run
 // slowly: with fewer than about 12 the same instructions took up to three
 // times as many cycles, so 4096 columns at 4 to a wave took 1.6 ms with the
 // other lanes off and 0.57 ms with them repeating columns.)
 template <typename T, typename IDX, bool ICE, bool PSEUDO, bool STATS, bool LEVELS = false,
-          bool FEW = false>
+          int LOOP = LOOP_LARGE>
 __global__ void __launch_bounds__(256) cape_grid_kernel(CapeGridArgs a, int cpw)
 {
     int64_t col;
     bool own = true;   // this lane stores its column's outputs
-    if constexpr (FEW) {
+    if constexpr (LOOP == LOOP_FEW) {
         const int lane = threadIdx.x & 63;
         const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * cpw;
         if (first >= a.ncol) return;
@@ -217,7 +217,7 @@ __global__ void __launch_bounds__(256) cape_grid_kernel(CapeGridArgs a, int cpw)
         ColumnOut<T> o;
         if (c.ts > 0.0f) {
             ran = true;
-            cape_column<T, XC_MATH, ICE, PSEUDO, SigmaCol<IDX>, NoLog, LEVELS, FEW>(
+            cape_column<T, XC_MATH, ICE, PSEUDO, SigmaCol<IDX>, NoLog, LEVELS, LOOP>(
                 c, nk, T(a.pinc), a.source, T(a.ml_depth), o, st);
         } else {
             o.cape = T(0); o.cin = T(0); o.zout = T(0); o.mulvl = 0;
@@ -629,35 +629,29 @@ hipError_t launch_srh(const CapeGridArgs &a, dim3 grid, int block, hipStream_t s
 // bytes, it is as fast at 110 000, and the pseudo-liquid one 3 % slower).
 inline int few_columns(int64_t ncol, bool fast_reversible_liquid)
 {
-    static const int simds = [] {
-        int dev = 0, ncu = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-        return 4 * (ncu > 0 ? ncu : 256);
-    }();
-    if (ncol > (int64_t)(fast_reversible_liquid ? 4 : 2 * 64) * simds) return 0;
-    const int64_t c = (ncol + simds - 1) / simds;
+    if (!few_waves(ncol, fast_reversible_liquid ? 2 : 64)) return 0;
+    const int64_t c = (ncol + device_simds() - 1) / device_simds();
     return c < 64 ? (int)c : 64;
 }
 
-template <typename T, typename IDX, bool STATS, bool LEVELS, bool FEW>
+template <typename T, typename IDX, bool STATS, bool LEVELS, int LOOP>
 hipError_t launch_cape_s(const CapeGridArgs &a, int block, int cpw, hipStream_t s)
 {
-    if (FEW) block = 256;
-    const int per = FEW ? 4 * cpw : block;
+    if (LOOP == LOOP_FEW) block = 256;
+    const int per = LOOP == LOOP_FEW ? 4 * cpw : block;
     const dim3 grid((unsigned)((a.ncol + per - 1) / per));
     switch (a.adiabat) {
     case 1:
-        cape_grid_kernel<T, IDX, false, true, STATS, LEVELS, FEW><<<grid, block, 0, s>>>(a, cpw);
+        cape_grid_kernel<T, IDX, false, true, STATS, LEVELS, LOOP><<<grid, block, 0, s>>>(a, cpw);
         break;
     case 2:
-        cape_grid_kernel<T, IDX, false, false, STATS, LEVELS, FEW><<<grid, block, 0, s>>>(a, cpw);
+        cape_grid_kernel<T, IDX, false, false, STATS, LEVELS, LOOP><<<grid, block, 0, s>>>(a, cpw);
         break;
     case 3:
-        cape_grid_kernel<T, IDX, true, true, STATS, LEVELS, FEW><<<grid, block, 0, s>>>(a, cpw);
+        cape_grid_kernel<T, IDX, true, true, STATS, LEVELS, LOOP><<<grid, block, 0, s>>>(a, cpw);
         break;
     case 4:
-        cape_grid_kernel<T, IDX, true, false, STATS, LEVELS, FEW><<<grid, block, 0, s>>>(a, cpw);
+        cape_grid_kernel<T, IDX, true, false, STATS, LEVELS, LOOP><<<grid, block, 0, s>>>(a, cpw);
         break;
     default: return hipErrorInvalidValue;
     }
@@ -667,13 +661,16 @@ hipError_t launch_cape_s(const CapeGridArgs &a, int block, int cpw, hipStream_t 
 template <typename T, typename IDX, bool STATS, bool LEVELS>
 hipError_t launch_cape_f(const CapeGridArgs &a, int block, hipStream_t s)
 {
-    // the counted launches keep the large grids' loop
+    const bool frl = XC_MATH == MATH_FAST && a.adiabat == 2;
+    const int cpw = few_columns(a.ncol, frl);
     if constexpr (!STATS) {
-        const bool frl = XC_MATH == MATH_FAST && a.adiabat == 2;
-        if (const int cpw = few_columns(a.ncol, frl))
-            return launch_cape_s<T, IDX, STATS, LEVELS, true>(a, block, cpw, s);
+        if (cpw) return launch_cape_s<T, IDX, STATS, LEVELS, LOOP_FEW>(a, block, cpw, s);
+    } else if constexpr (sizeof(T) == 4 && XC_MATH == MATH_ACCURATE) {
+        // the counted launches keep the large grids' columns, one to a lane,
+        // and their masks
+        if (cpw) return launch_cape_s<T, IDX, STATS, LEVELS, LOOP_MASKS>(a, block, 0, s);
     }
-    return launch_cape_s<T, IDX, STATS, LEVELS, false>(a, block, 0, s);
+    return launch_cape_s<T, IDX, STATS, LEVELS, LOOP_LARGE>(a, block, 0, s);
 }
 
 // 32-bit element offsets when every index of the profile arrays fits (the
@@ -708,14 +705,11 @@ template <bool ICE, bool PSEUDO, bool PREDICT, bool STATS, bool LEVELS>
 int ascent_grid(int block, int64_t ncol, int *cpw)
 {
     static int per_cu[5] = {-1, -1, -1, -1, -1};   // by block / 64
-    static int ncu = 0;
     const int slot = block / 64;
     *cpw = 64;
     if (slot < 1 || slot > 4) return 1;
     if (per_cu[slot] < 0) {
-        int dev = 0, pc = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+        int pc = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
                 &pc, reinterpret_cast<const void *>(
                          warm_ascent_kernel<ICE, PSEUDO, PREDICT, STATS, LEVELS>),
@@ -724,7 +718,7 @@ int ascent_grid(int block, int64_t ncol, int *cpw)
             pc = 1;
         per_cu[slot] = pc;
     }
-    const int64_t cus = ncu > 0 ? ncu : 1, simds = 4 * cus;
+    const int64_t simds = device_simds();
     if (!STATS && ncol < 64 * simds) *cpw = (int)((ncol + simds - 1) / simds);
     const int64_t cols = (int64_t)*cpw * slot;   // a block's columns
     int64_t g = (ncol + cols - 1) / cols;
@@ -733,7 +727,7 @@ int ascent_grid(int block, int64_t ncol, int *cpw)
     // ascent for one of them (121 x 97 columns: 961 us with 40 blocks, 713
     // with 48, 64 columns to a wave)
     if (g > (int64_t)WORK_PARTS) g = (g + WORK_PARTS - 1) / WORK_PARTS * WORK_PARTS;
-    const int64_t full = cus * per_cu[slot];
+    const int64_t full = simds / 4 * per_cu[slot];
     if (g > full) g = full >= (int64_t)WORK_PARTS ? full - full % WORK_PARTS : full;
     return (int)g;
 }

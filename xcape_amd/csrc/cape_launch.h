@@ -70,6 +70,25 @@ inline int64_t warm_scratch_floats(int64_t nk_in, bool levels)
     return 4 * (nk_in + 1) + (levels ? nk_in + 1 : 0) + 16;
 }
 
+// The device's SIMDs, four to a CU.
+inline int device_simds()
+{
+    static const int simds = [] {
+        int dev = 0, ncu = 0;
+        (void)hipGetDevice(&dev);
+        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+        return 4 * (ncu > 0 ? ncu : 256);
+    }();
+    return simds;
+}
+
+// A plain launch of so many waves (cpw columns to each) takes the loops for
+// few waves: at most two per SIMD.
+inline bool few_waves(int64_t ncol, int cpw)
+{
+    return ncol <= (int64_t)2 * cpw * device_simds();
+}
+
 // kind of work a grid launch does
 enum { GRID_CAPE = 1, GRID_SRH = 2, GRID_CAPE_SRH = 3 };
 

@@ -191,8 +191,12 @@ __global__ void reset_counters(unsigned int *c)
 }
 
 // The reference's loops (cape_column).  TILED: stage the first a.tile levels
-// in LDS.  STATS: accumulate the work counters.
-template <int MATH, bool ICE, bool PSEUDO, bool TILED, bool STATS>
+// in LDS.  STATS: accumulate the work counters.  LOOP: solve_raw's, LOOP_FEW
+// for a batch of few waves, where a wave has its SIMD nearly to itself and
+// waits for the large loop's votes and masks (mixed batches of 30 to 137
+// levels: 2000 columns 2440 us with the large loop, 1840 so; 64 000, 2635 and
+// 2155; 130 000, 2915 and 2420).
+template <int MATH, bool ICE, bool PSEUDO, bool TILED, bool STATS, int LOOP>
 __global__ void __launch_bounds__(256) ragged_kernel(RaggedArgs a)
 {
     // LDS: per wave, 3 arrays x tile levels x 64 lanes, level-major so the
@@ -250,7 +254,8 @@ __global__ void __launch_bounds__(256) ragged_kernel(RaggedArgs a)
             ColumnOut<float> o{};
             const int nk = nk_in + 1;
             const int src = a.src_sorted[j];
-            cape_column<float, MATH, ICE, PSEUDO>(c, nk, a.pinc, src, a.ml_depth, o, st);
+            cape_column<float, MATH, ICE, PSEUDO, Col, NoLog, false, LOOP>(c, nk, a.pinc, src,
+                                                                           a.ml_depth, o, st);
             a.mulvl[col] = o.mulvl;
             a.cape[col] = o.cape;
             a.cin[col] = o.cin;
@@ -271,31 +276,33 @@ __global__ void __launch_bounds__(256) ragged_kernel(RaggedArgs a)
 
 using Kernel = void (*)(RaggedArgs);
 
-template <int MATH, bool TILED, bool STATS>
+template <int MATH, bool TILED, bool STATS, int LOOP>
 Kernel pick_adiabat(int adiabat)
 {
     switch (adiabat) {
-    case 1: return ragged_kernel<MATH, false, true, TILED, STATS>;
-    case 2: return ragged_kernel<MATH, false, false, TILED, STATS>;
-    case 3: return ragged_kernel<MATH, true, true, TILED, STATS>;
-    default: return ragged_kernel<MATH, true, false, TILED, STATS>;
+    case 1: return ragged_kernel<MATH, false, true, TILED, STATS, LOOP>;
+    case 2: return ragged_kernel<MATH, false, false, TILED, STATS, LOOP>;
+    case 3: return ragged_kernel<MATH, true, true, TILED, STATS, LOOP>;
+    default: return ragged_kernel<MATH, true, false, TILED, STATS, LOOP>;
     }
 }
 
-template <int MATH>
-Kernel pick_math(int adiabat, bool tiled, bool stats)
+template <int MATH, int LOOP>
+Kernel pick_loop(int adiabat, bool tiled, bool stats)
 {
-    if (tiled) return stats ? pick_adiabat<MATH, true, true>(adiabat)
-                            : pick_adiabat<MATH, true, false>(adiabat);
-    return stats ? pick_adiabat<MATH, false, true>(adiabat)
-                 : pick_adiabat<MATH, false, false>(adiabat);
+    if (tiled) return stats ? pick_adiabat<MATH, true, true, LOOP>(adiabat)
+                            : pick_adiabat<MATH, true, false, LOOP>(adiabat);
+    return stats ? pick_adiabat<MATH, false, true, LOOP>(adiabat)
+                 : pick_adiabat<MATH, false, false, LOOP>(adiabat);
 }
 
-// the plain method's kernel for one segment
-Kernel pick(bool fast, int adiabat, bool tiled, bool stats)
+// the plain method's kernel for one segment; few: the batch's waves are few
+// (fast math has one loop)
+Kernel pick(bool fast, int adiabat, bool tiled, bool stats, bool few)
 {
-    return fast ? pick_math<MATH_FAST>(adiabat, tiled, stats)
-                : pick_math<MATH_ACCURATE>(adiabat, tiled, stats);
+    if (fast) return pick_loop<MATH_FAST, LOOP_LARGE>(adiabat, tiled, stats);
+    return few ? pick_loop<MATH_ACCURATE, LOOP_FEW>(adiabat, tiled, stats)
+               : pick_loop<MATH_ACCURATE, LOOP_LARGE>(adiabat, tiled, stats);
 }
 
 }  // namespace
@@ -318,6 +325,7 @@ struct xcape_ragged_plan {
     int block = 256;
     size_t lds_bytes = 0;
     bool fast = false, warm = false;
+    bool few = false;                  // plain plans: the batch's waves are few
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
 };
@@ -358,7 +366,7 @@ hipError_t enqueue(const xcape_ragged_plan *pl, bool stats, hipStream_t s,
             a.seg_end = pl->seg_end[g];
             a.counter = pl->d_counter + g;
             a.stats = stats ? pl->d_stats : nullptr;
-            const Kernel k = pick(pl->fast, g + 1, pl->args.tile > 0, stats);
+            const Kernel k = pick(pl->fast, g + 1, pl->args.tile > 0, stats, pl->few);
             void *kargs[] = {&a};
             e = hipLaunchKernel(reinterpret_cast<const void *>(k), dim3(pl->seg_grid[g]),
                                 dim3(pl->block), kargs, pl->lds_bytes, sg);
@@ -500,6 +508,8 @@ int xcape_ragged_plan_create(const int64_t *offsets_host, const int32_t *source_
     a.cape = cape; a.cin = cin; a.zout = zmulev; a.mulvl = mulev;
     a.chunk = chunk; a.tile = tile;
     a.cpw = cols_per_block < 64 ? cols_per_block : 64;
+    // (the segments run beside each other: the whole batch's waves)
+    pl->few = few_waves(ncol, a.cpw);
     if (pl->warm) {
         // each segment as a grid of its own for the warm kernels: its columns
         // start seg_begin into each level row of the staged copies
@@ -551,7 +561,7 @@ int xcape_ragged_plan_create(const int64_t *offsets_host, const int32_t *source_
         int per_cu = 0;
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
             &per_cu,
-            reinterpret_cast<const void *>(pick(pl->fast, g + 1, tile > 0, false)),
+            reinterpret_cast<const void *>(pick(pl->fast, g + 1, tile > 0, false, pl->few)),
             pl->block, pl->lds_bytes);
         if (e != hipSuccess || per_cu < 1) per_cu = 1;
         // enough blocks to fill every CU once, never more than the work needs

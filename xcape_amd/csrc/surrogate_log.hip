@@ -14,6 +14,7 @@
 #include "../../include/xcape_hip.h"
 #include "capi_common.h"
 #include "cape_column.h"
+#include "cape_launch.h"
 
 using namespace xcape;
 
@@ -61,7 +62,7 @@ struct SampleLogger {
     }
 };
 
-template <bool ICE, bool PSEUDO>
+template <bool ICE, bool PSEUDO, int LOOP>
 __global__ void __launch_bounds__(256) log_kernel(const float *p, const float *t,
                                                   const float *td, const float *ps,
                                                   const float *ts, const float *tds, int nk_in,
@@ -74,8 +75,18 @@ __global__ void __launch_bounds__(256) log_kernel(const float *p, const float *t
     LaneStats st;
     ColumnOut<float> o;
     lg.col = col;
-    cape_column<float, MATH_ACCURATE, ICE, PSEUDO>(c, nk_in + 1, pinc, source, ml_depth, o, st,
-                                                   lg);
+    cape_column<float, MATH_ACCURATE, ICE, PSEUDO, LogCol, SampleLogger, false, LOOP>(
+        c, nk_in + 1, pinc, source, ml_depth, o, st, lg);
+}
+
+template <int LOOP> auto pick(int adiabat)
+{
+    switch (adiabat) {
+    case 1: return log_kernel<false, true, LOOP>;
+    case 2: return log_kernel<false, false, LOOP>;
+    case 3: return log_kernel<true, true, LOOP>;
+    default: return log_kernel<true, false, LOOP>;
+    }
 }
 
 }  // namespace
@@ -102,12 +113,8 @@ extern "C" int xcape_surrogate_log_f32(const float *p, const float *t, const flo
     if (keep_fraction >= 1.0f) lg.keep = 0x10000u;
     hipStream_t s = (hipStream_t)stream;
     dim3 grid((unsigned)((ncol + 255) / 256));
-    switch (adiabat) {
-    case 1: log_kernel<false, true><<<grid, 256, 0, s>>>(p, t, td, ps, ts, tds, (int)nk, ncol, pinc, source, ml_depth, lg); break;
-    case 2: log_kernel<false, false><<<grid, 256, 0, s>>>(p, t, td, ps, ts, tds, (int)nk, ncol, pinc, source, ml_depth, lg); break;
-    case 3: log_kernel<true, true><<<grid, 256, 0, s>>>(p, t, td, ps, ts, tds, (int)nk, ncol, pinc, source, ml_depth, lg); break;
-    default: log_kernel<true, false><<<grid, 256, 0, s>>>(p, t, td, ps, ts, tds, (int)nk, ncol, pinc, source, ml_depth, lg); break;
-    }
+    const auto k = few_waves(ncol, 64) ? pick<LOOP_FEW>(adiabat) : pick<LOOP_LARGE>(adiabat);
+    k<<<grid, 256, 0, s>>>(p, t, td, ps, ts, tds, (int)nk, ncol, pinc, source, ml_depth, lg);
     hipError_t e = hipGetLastError();
     return e ? hip_fail(e, "surrogate log") : XCAPE_OK;
 }
