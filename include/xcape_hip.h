@@ -106,7 +106,8 @@ int xcape_device_count(void);
 /*
  * Host-array calls (no XCAPE_DEVICE_PTRS, column-contiguous arrays, double
  * ones included) stream their columns in chunks of about 128 MB of input
- * (XCAPE_HOST_CHUNK_MB; up to 64 MB go as one chunk) through pinned host memory and device buffers that stay allocated for the
+ * (XCAPE_HOST_CHUNK_MB; small calls, up to 32 to 64 MB, go as one chunk)
+ * through pinned host memory and device buffers that stay allocated for the
  * next call: at most two such staging sets per process (three slots of
  * pinned input, pinned output and device buffers each), so at most two
  * host-array calls stream at once and a third waits for one of them.  This

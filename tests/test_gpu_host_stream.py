@@ -203,3 +203,25 @@ def test_out_of_core_memmap(hip, tmp_path):
     for a, b in zip(got, ref):
         assert a.shape == (60, 100)
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize('ncol', [17476, 17477, 36000, 58000])
+def test_streamed_in_groups_of_arrays(hip, monkeypatch, ncol):
+    """A chunk's arrays go up one by one, or, from 4 MB an array (17 477
+    columns of 60 levels), in groups of at least 8 MB, small arrays with the
+    profile before them: on both sides of the limit, in one chunk and (58 000
+    columns, over 64 MB with the winds) in several, the device call's results
+    bit for bit."""
+    monkeypatch.delenv('XCAPE_HOST_CHUNK_MB', raising=False)
+    c = synthetic.sigma_columns_torch(ncol, NK, 12)
+    rng = np.random.default_rng(4)
+    wind = {k: rng.normal(5.0, 8.0, (ncol, NK)).astype(np.float32) for k in ('u', 'v')}
+    wind.update({k + 's': rng.normal(2.0, 4.0, ncol).astype(np.float32) for k in ('u', 'v')})
+    prof = [c[k].cpu().numpy() for k in ('p', 't', 'td')]
+    sfc = [c[k].cpu().numpy() for k in ('ps', 'ts', 'tds')]
+    args = prof + [wind['u'], wind['v']] + sfc + [wind['us'], wind['vs']]
+    _same(hip.srh(*args), hip.srh(*_dev(args)))
+    kw = dict(source=2, adiabat=1, fast_math=True, pinc=2500.)
+    _same(hip.cape_srh(*args, **kw), hip.cape_srh(*_dev(args), **kw))
+    shared = [np.linspace(1000.0, 100.0, NK).astype(np.float32)] + args[1:]
+    _same(hip.srh(*shared, p_shared=True), hip.srh(*_dev(shared), p_shared=True))

@@ -557,26 +557,43 @@ struct GridCall {
 //     area each) run the chunk's kernels once its upload has ended, download
 //     its outputs, and are drained into the caller's arrays when the calling
 //     thread comes back to the slot.
-// A call of up to STAGE_WHOLE_MB of input goes as one chunk.  An ascent's
+// A call of up to stage_whole_mb() of input goes as one chunk.  An ascent's
 // kernel takes 0.6 to 1.4 ms for few columns as for a device full, longer than
 // such an upload, and chunks whose streams share a hardware queue wait for each
 // other.  In one chunk / a quarter, a half and the rest (median us, 8 threads):
 // 40 levels, surface, 2 MB 688 / 1635, 24 MB 1365 / 1792, 64 MB 2900 / 2994,
 // 107 MB 4198 / 3526; 137 levels, most unstable, pseudo-ice, 2 MB 1246 / 2222,
-// 24 MB 2222 / 3602, 64 MB 3127 / 4436, 107 MB 4883 / 4737.  Larger calls start
-// with a quarter and a half of a chunk, so that the first upload and the first
-// kernels start early.  A chunk of an array is one contiguous range of the
-// caller's array and one contiguous run of the staging areas.
+// 24 MB 2222 / 3602, 64 MB 3127 / 4436, 107 MB 4883 / 4737.  An ascent of more
+// columns than two waves per SIMD takes longer the more there are, and its
+// chunks pay from about 50 MB on (37 shared levels, surface, 210 000 columns of
+// 65 MB 3517 / 2778, 166 666 of 51 MB 2829 / 2627; 20 levels, most unstable,
+// pseudo-ice, 300 000 of 52 MB 4886 / 5209).  The helicity chain's kernel is
+// short, and the upload is what chunks hide: 32 MB (30 shared levels, 36 MB
+// 1216 / 1164, 63 MB 1951 / 1799; 60 levels, 24 MB 813 / 898, 63 MB 1693 /
+// 1738).  Larger calls start with a quarter and a half of a chunk, so that the
+// first upload and the first kernels start early.  A chunk of an array is one
+// contiguous range of the caller's array and one contiguous run of the staging
+// areas.
 
 constexpr int STAGE_IN = 3;
 constexpr int STAGE_SLOTS = 4;
 constexpr int STAGE_SETS = 2;   // at most this many calls stream at once; others wait
-constexpr size_t STAGE_WHOLE_MB = 64;
 // bytes of a chunk that goes in one upload; the arrays of a larger one go one by
 // one, each while the next is copied (64 MB in one chunk, 40 levels: 2900 us
-// against 3152; 137 levels: 3127 against 3400)
+// against 3152; 137 levels: 3127 against 3400), or, where several threads copy
+// an array, in groups of at least STAGE_GROUP: starting the threads takes about
+// as long as 4 MB of copying (helicity chain, 60 levels, 24 MB 813 us, 72 MB
+// 1945, against 1110 and 2743 array by array; arrays of less than
+// COPY_ONE_THREAD are better alone, 17 MB of 3.4 MB arrays 748 us against 772)
 constexpr size_t STAGE_ONE_UPLOAD = (size_t)2 << 20;
+constexpr size_t COPY_ONE_THREAD = (size_t)4 << 20;
+constexpr size_t STAGE_GROUP = (size_t)8 << 20;
 constexpr size_t STAGE_ALIGN = 256;
+
+size_t stage_whole_mb(int64_t ncol, bool want_cape)
+{
+    return !want_cape ? 32 : few_waves(ncol, 64) ? 64 : 50;
+}
 
 size_t align_up(size_t x) { return (x + STAGE_ALIGN - 1) / STAGE_ALIGN * STAGE_ALIGN; }
 
@@ -621,7 +638,7 @@ void parallel_copy(const CopyJob *jobs, int njobs, int threads)
 {
     size_t total = 0;
     for (int j = 0; j < njobs; ++j) total += jobs[j].n;
-    if (total < ((size_t)4 << 20)) threads = 1;
+    if (total < COPY_ONE_THREAD) threads = 1;
     const size_t per = (total + threads - 1) / (size_t)threads;
     auto share = [jobs, njobs, total, per](int t) {
         const size_t lo = (size_t)t * per, hi = lo + per < total ? lo + per : total;
@@ -826,7 +843,8 @@ int stream_host_grid(const GridCall &c, const CapeGridArgs &tmpl, bool want_cape
     // columns per chunk: about XCAPE_HOST_CHUNK_MB of input, a multiple of 64
     int64_t m = ((int64_t)host_chunk_mb() << 20) / (int64_t)in_col / 64 * 64;
     if (m < 64) m = 64;
-    const bool whole = (size_t)ncol * in_col <= (STAGE_WHOLE_MB << 20) && m >= ncol;
+    const bool whole = (size_t)ncol * in_col <= (stage_whole_mb(ncol, want_cape) << 20) &&
+                       m >= ncol;
     if (m > ncol) m = ncol;
     size_t off_in[12], off_out[12];
     const size_t in_bytes = in.place(m, off_in), out_bytes = out.place(m, off_out);
@@ -909,11 +927,13 @@ int stream_host_grid(const GridCall &c, const CapeGridArgs &tmpl, bool want_cape
             if (pend[sl].busy) XC_TRY(drain(sl));
             XC_TRY(hipMemcpyAsync(din, st->pin_in[r], ib, hipMemcpyHostToDevice, st->up));
         } else {
-            // each profile array by itself, the small ones between them together
+            // a profile array with the small ones behind it, or several to a group
+            const size_t group = whole && prof * (size_t)n < COPY_ONE_THREAD ? 0 : STAGE_GROUP;
             for (int i = 0, e1; i < in.count; i = e1) {
+                size_t bytes = in.bytes(i, n);
                 e1 = i + 1;
-                if (in.cb[i] != prof)
-                    while (e1 < in.count && in.cb[e1] != prof) ++e1;
+                while (e1 < in.count && (in.cb[e1] != prof || bytes < group))
+                    bytes += in.bytes(e1++, n);
                 parallel_copy(jobs + i, e1 - i, threads);
                 if (i == 0 && pend[sl].busy) XC_TRY(drain(sl));
                 const size_t end = e1 < in.count ? oi[e1] : ib;
