@@ -682,21 +682,26 @@ struct StagingSet {
     hipStream_t stream[STAGE_SLOTS] = {};     // a slot's kernels and download
     hipEvent_t done[STAGE_SLOTS] = {};        // a slot's last download
 
-    void free_pinned()
+    // pinned buffers of at least `need` bytes each (0: freed)
+    template <size_t N> static hipError_t grow(char *(&bufs)[N], size_t &cap, size_t need)
     {
-        for (auto &x : pin_in) {
+        if (need != 0 && need <= cap) return hipSuccess;
+        cap = 0;
+        for (auto &x : bufs) {
             if (x) (void)hipHostFree(x);
             x = nullptr;
         }
-        for (auto &x : pin_out) {
-            if (x) (void)hipHostFree(x);
-            x = nullptr;
-        }
-        in_cap = out_cap = 0;
+        hipError_t e;
+        if (need)
+            for (auto &x : bufs)
+                if ((e = hipHostMalloc((void **)&x, need, hipHostMallocDefault))) return e;
+        cap = need;
+        return hipSuccess;
     }
     void destroy()
     {
-        free_pinned();
+        (void)grow(pin_in, in_cap, 0);
+        (void)grow(pin_out, out_cap, 0);
         if (dev) (void)hipFree(dev);
         dev = nullptr;
         dev_cap = 0;
@@ -729,15 +734,9 @@ struct StagingSet {
                 return e;
             if (!done[i] && (e = hipEventCreateWithFlags(&done[i], ev))) return e;
         }
-        if (in > in_cap || out > out_cap) {
-            free_pinned();
-            for (auto &x : pin_in)
-                if ((e = hipHostMalloc((void **)&x, in, hipHostMallocDefault))) return e;
-            for (auto &x : pin_out)
-                if ((e = hipHostMalloc((void **)&x, out, hipHostMallocDefault))) return e;
-            in_cap = in;
-            out_cap = out;
-        }
+        // (each by itself, and never smaller: calls of different shapes take turns
+        // on one set, and pinning its buffers takes longer than they do)
+        if ((e = grow(pin_in, in_cap, in)) || (e = grow(pin_out, out_cap, out))) return e;
         if (devb > dev_cap) {
             if (dev) (void)hipFree(dev);
             dev = nullptr;
