@@ -375,8 +375,10 @@ int xcape_surrogate_log_f32(const float *p, const float *t, const float *td,
  * (n,) -> y (n,), for checking its rounding on the device at hand: fn 0 the
  * raw IEEE division kernel, 1 the compiler's IEEE division, 2 division by a
  * per-call constant (its reciprocal rounded once), 3 the exp kernel, 4 the
- * device library's expf, 5 the pow kernel, 6 the device library's powf.
- * b is unused (may be NULL) for fn 3 and 4.  Asynchronous on `stream`.
+ * device library's expf, 5 the pow kernel, 6 the device library's powf, 7 the
+ * reciprocal the division starts from, 8 the exp kernel for small arguments
+ * (|a| < 0.34), 9 the log kernel, 10 the device library's logf.  b is unused
+ * (may be NULL) but for fn 0, 1, 2, 5 and 6.  Asynchronous on `stream`.
  * No reference counterpart.
  */
 int xcape_math_check(int fn, const float *a, const float *b, int64_t n, float *y,

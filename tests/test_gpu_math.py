@@ -224,3 +224,64 @@ def test_raw_division_f64_is_ieee(dev):
                    [3.0, np.nan]])
     assert np.isnan(H.math_check_f64(4, torch.from_numpy(sp).cuda()).cpu().numpy()).all()
 
+
+
+def _floats(torch, lo, hi, step=1 << 26):
+    """Every float from lo to hi (positive, lo < hi), in device tensors."""
+    lo, hi = (int(np.float32(x).view(np.int32)) for x in (lo, hi))
+    for i in range(lo, hi + 1, step):
+        yield torch.arange(i, min(i + step, hi + 1), dtype=torch.int32,
+                           device='cuda').view(torch.float32)
+
+
+def _differ(torch, a, b):
+    return int(torch.count_nonzero(a.view(torch.int32) != b.view(torch.int32)))
+
+
+def test_reciprocal_is_correctly_rounded(dev):
+    """The premise of the division's single correction: the reciprocal it
+    starts from is the IEEE 1 / b, for every mantissa at exponents from 2^-97
+    to 2^73, both signs."""
+    torch, H = dev
+    m = torch.arange(1 << 23, dtype=torch.int32, device='cuda')
+    for e in (-97, -60, -20, 0, 17, 41, 73):
+        for sign in (0, -(1 << 31)):
+            b = (m + ((e + 127) << 23) + sign).view(torch.float32)
+            assert _differ(torch, H.math_check(7, b), H.math_check(1, torch.ones_like(b), b)) == 0
+    sp = torch.tensor([0.0, float('inf'), float('nan')], device='cuda')
+    assert bool(torch.isnan(H.math_check(7, sp)).all())
+
+
+def test_raw_division_near_ties(dev):
+    """Quotients whose remainder is the smallest there is: a = q b rounded, and
+    its neighbours, for q next to a rounding boundary."""
+    torch, H = dev
+    g = torch.Generator(device='cuda')
+    g.manual_seed(3)
+    n = 1 << 22
+    for _ in range(8):
+        q = 1.0 + torch.rand(n, generator=g, device='cuda', dtype=torch.float64)
+        half = torch.floor(q * 2.0 ** 23) / 2.0 ** 23 + 2.0 ** -24     # between two floats
+        b = (1.0 + torch.rand(n, generator=g, device='cuda')).float()
+        a = (half * b.double()).float()
+        for k in (-1, 0, 1):
+            ak = (a.view(torch.int32) + k).view(torch.float32)
+            assert _differ(torch, H.math_check(0, ak, b), H.math_check(1, ak, b)) == 0
+
+
+def test_small_exp_equals_the_exp_kernel(dev):
+    torch, H = dev
+    for x in _floats(torch, 0.0, 0.34):
+        for y in (x, -x):
+            assert _differ(torch, H.math_check(8, y), H.math_check(3, y)) == 0
+
+
+def test_log_kernel_equals_library_logf(dev):
+    """Every float from 1e-30 to 1e30: the log kernel is the device library's
+    logf bit for bit (the pressures' ratios are taken from 1e-26 to 1e26)."""
+    torch, H = dev
+    for x in _floats(torch, 1e-30, 1e30):
+        assert _differ(torch, H.math_check(9, x), H.math_check(10, x)) == 0
+    sp = torch.tensor([0.0, -1.0, -1e-20, float('nan')], device='cuda')
+    assert bool(torch.isnan(H.math_check(9, sp)).all())
+    assert float(H.math_check(9, torch.ones(1, device='cuda'))) == 0.0

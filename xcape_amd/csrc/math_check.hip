@@ -4,7 +4,8 @@
 //
 // fn: 0 div_raw(a, b)   1 a / b (the compiler's IEEE division)
 //     2 div_const(a, b, RN(1/b))   3 exp_core(a)   4 expf(a)
-//     5 pow_core(a, b)   6 powf(a, b)
+//     5 pow_core(a, b)   6 powf(a, b)   7 rcp_rn(a)   8 exp_small(a)
+//     9 log_core(a)   10 logf(a)
 // xcape_math_check_f64: fn 0 log_core_f64(a)   1 log(a)   2 exp_core_f64(a)
 //     3 exp(a)   4 ddiv_raw(a0, a1)   5 a0 / a1 (FP64; a holds the pairs)
 #include <hip/hip_runtime.h>
@@ -31,7 +32,11 @@ __global__ void math_check_kernel(int fn, const float *a, const float *b, int64_
     case 3: r = exp_core(x); break;
     case 4: r = expf(x); break;
     case 5: r = pow_core(x, z); break;
-    default: r = powf(x, z); break;
+    case 6: r = powf(x, z); break;
+    case 7: r = rcp_rn(x); break;
+    case 8: r = exp_small(x); break;
+    case 9: r = log_core(x); break;
+    default: r = logf(x); break;
     }
     y[i] = r;
 }
@@ -55,9 +60,9 @@ __global__ void math_check_f64_kernel(int fn, const double *a, int64_t n, double
 extern "C" int xcape_math_check(int fn, const float *a, const float *b, int64_t n, float *y,
                                 void *stream)
 {
-    if (fn < 0 || fn > 6) return fail(XCAPE_EINVAL, "fn=%d not in 0..6", fn);
+    if (fn < 0 || fn > 10) return fail(XCAPE_EINVAL, "fn=%d not in 0..10", fn);
     if (n < 0 || n > ((int64_t)1 << 31)) return fail(XCAPE_EINVAL, "n=%lld out of range", (long long)n);
-    const bool binary = fn <= 2 || fn >= 5;
+    const bool binary = fn <= 2 || fn == 5 || fn == 6;
     if (!a || !y || (binary && !b)) return fail(XCAPE_EINVAL, "NULL argument");
     int rc = ensure_device();
     if (rc) return rc;

@@ -66,15 +66,16 @@ template <> struct Phys<double> {
 // Division: the correctly rounded quotient by Markstein's theorem: with y the
 // correctly rounded 1/b, q = RN(a y) and one correction by the exact residual
 // a - b q (fma) give RN(a/b).  The hardware reciprocal with one Newton step
-// is the correctly rounded one: compared on the device with IEEE 1/b over
-// every 23-bit mantissa at seven exponents from 2^-97 to 2^73, none differs
-// (the quotient has one correction fewer than the compiler's sequence, which
-// allows for an inexact reciprocal; 8.6e9 random quotients, none differs).
+// is the correctly rounded one: equal on the device to IEEE 1/b over every
+// 23-bit mantissa at seven exponents from 2^-97 to 2^73 (the quotient has one
+// correction fewer than the compiler's sequence, which allows for an inexact
+// reciprocal).
 // So for a, b and a/b normal, |b| < 2^126, the result is the IEEE quotient
 // bit for bit.  A zero, infinite or NaN operand (a zero dividend apart) gives
 // NaN; subnormal or huge operands give a wrong value.  Callers make sure of
-// the range (the fixed-point evaluation re-evaluates with IEEE division
-// whenever its result is not finite).
+// the range (a sub-step whose exponents leave theirs is solved again with IEEE
+// division; the interpolations of the helicity chain take it where the quotient
+// is not finite).
 __device__ __forceinline__ float rcp_rn(float b)
 {
     const float y0 = __builtin_amdgcn_rcpf(b);
@@ -131,8 +132,8 @@ __device__ __forceinline__ float exp_core(float x)
 }
 
 // exp(x) for |x| < EXP_SMALL_MAX: exp_core's nearest integer is 0 there, so
-// its reduction and scaling drop out (exp_core's value bit for bit: compared
-// over every such float on the device).
+// its reduction and scaling drop out (exp_core's value bit for bit over every
+// such float).
 constexpr float EXP_SMALL_MAX = 0.34f;   // 0.34 log2(e) < 1/2
 
 __device__ __forceinline__ float exp_small(float x)
@@ -148,8 +149,8 @@ __device__ __forceinline__ float exp_small(float x)
 // ln x: the hardware log2 times ln 2 as a double-float (ln 2's bit patterns
 // 0x3f317217, 0x3377d1cf), the device library's steps without its scaling of
 // subnormals and its infinity select: the library's value for every float
-// from 1e-30 to 1e30 (compared over all of them on the device); -inf for 0,
-// NaN for a negative or NaN x.
+// from 1e-30 to 1e30 (compared over all of them on the device); NaN for
+// a zero, negative or NaN x.
 __device__ __forceinline__ float log_core(float x)
 {
     constexpr float LN2 = 0x1.62e42ep-1f;
