@@ -146,20 +146,17 @@ __device__ __forceinline__ float exp_small(float x)
     return __builtin_amdgcn_exp2f(ph + pl);
 }
 
-// ln x: the hardware log2 times ln 2 as a double-float (ln 2's bit patterns
-// 0x3f317217, 0x3377d1cf), the device library's steps without its scaling of
-// subnormals and its infinity select: the library's value for every float
-// from 1e-30 to 1e30 (compared over all of them on the device); NaN for
-// a zero, negative or NaN x.
+// ln x = l ln 2 with l the hardware's log2 x.  ln 2 is HI + LO to 2^-54, HI
+// the nearest float and LO what is left; RN(l HI + RN(l LO)) is l ln 2 rounded
+// but for 2^-25 ulp (l LO is below 2^-27 of the product, and its own rounding
+// the only other one).  The device library's logf for every float from 1e-30
+// to 1e30; NaN for a zero, negative or NaN x.
 __device__ __forceinline__ float log_core(float x)
 {
-    constexpr float LN2 = 0x1.62e42ep-1f;
-    constexpr float LN2_LO = 0x1.efa39ep-25f;
+    constexpr double LN2 = 0.693147180559945309417;
+    constexpr float HI = (float)LN2, LO = (float)(LN2 - HI);
     const float l = __builtin_amdgcn_logf(x);
-    const float h = l * LN2;
-    float r = __builtin_fmaf(l, LN2, -h);
-    r = __builtin_fmaf(l, LN2_LO, r);
-    return h + r;
+    return __builtin_fmaf(l, HI, l * LO);
 }
 
 // x^y for 0 < x < 2^126, |y| <= 1 (the Exner function and theta-e's power):
