@@ -261,3 +261,47 @@ def test_profiles_where_they_lie_match_level_major(hip, ncol, nk, p_shared):
                 kw = dict(depth=depth, fp64=fp64, inputs_f64=dt == np.float64, p_shared=p_shared)
                 for x, y in zip(hip.srh(*a, **kw), hip.srh(*b, level_major=True, **kw)):
                     assert torch.equal(x.nan_to_num(nan=-7e7), y.nan_to_num(nan=-7e7))
+
+
+@pytest.mark.parametrize('p_shared', [False, True])
+@pytest.mark.parametrize('ncol,nk', [(128, 5), (700, 33), (3000, 137)])
+def test_combined_in_parts_matches_the_calls_apart(hip, monkeypatch, ncol, nk, p_shared):
+    """A warm-started combined call on 2^20 device columns or more is staged in
+    four parts and takes its helicity from level-major copies of the winds, a
+    lane per column; below, and alone, the helicity reads the profiles where
+    they lie.  Forced here down to 128 columns (3000: parts of 768, the last of
+    696): each output is the separate calls', bit for bit, with columns whose
+    heights fall, NaN and values that the slab kernel hands on."""
+    import torch
+    names = ('p', 't', 'td', 'u', 'v', 'ps', 'ts', 'tds', 'us', 'vs')
+    if p_shared:
+        c = synthetic.pressure_columns(ncol, ncol, levels=np.linspace(1000, 100, nk), winds=True)
+    else:
+        c = synthetic.sigma_columns(ncol, nk, ncol, winds=True)
+    if ncol > 500:
+        c['t'][5, 3] = np.nan
+        c['td'][7, nk // 2:] = np.nan
+        c['t'][9, nk - 3] = -300.0
+        c['td'][15, nk - 2] = 1000.0
+        c['u'][13, 4] = np.nan
+        if not p_shared:
+            c['p'][3] = c['p'][3][::-1]
+            c['p'][8, 20] = c['p'][8, 19]
+            c['p'][21, 25] = np.inf
+    a = [torch.from_numpy(np.ascontiguousarray(c[k])).cuda() for k in names]
+    kw = dict(pinc=500., source=2, adiabat=3, p_shared=p_shared, warm_start='extrapolation')
+    monkeypatch.delenv('XCAPE_STAGE_COLUMNS', raising=False)
+    monkeypatch.delenv('XCAPE_WARM_PIPE_COLUMNS', raising=False)
+    apart = hip.cape(*(x for k, x in zip(names, a) if k not in ('u', 'v', 'us', 'vs')), **kw)
+    apart += hip.srh(*a, depth=3000., p_shared=p_shared)
+    one = hip.cape_srh(*a, depth=3000., **kw)
+    monkeypatch.setenv('XCAPE_WARM_PIPE_COLUMNS', '128')
+    parts = hip.cape_srh(*a, depth=3000., **kw)
+    levels = hip.cape(*(x for k, x in zip(names, a) if k not in ('u', 'v', 'us', 'vs')),
+                      levels=True, **kw)
+    for x, y, z in zip(apart, one, parts):
+        x = x.nan_to_num(nan=-7e7)
+        assert torch.equal(y.nan_to_num(nan=-7e7), x)
+        assert torch.equal(z.nan_to_num(nan=-7e7), x)
+    for x, z in zip(apart[:4], levels):
+        assert torch.equal(z.nan_to_num(nan=-7e7), x.nan_to_num(nan=-7e7))
