@@ -7,7 +7,8 @@ motion on the same columns (xcape_cape_srh_f32).  Inputs are generated in HBM
 (seeded synthetic soundings and winds) before the timed region; outputs stay
 in HBM.
 
-Prints one JSON line:
+Prints one JSON line, its sections shortened; --detail FILE writes the line
+with them in full (accuracy, configs, ragged_200k, the kernels' counts):
   value         columns/s of the warm-started path (surrogate + extrapolation)
   plain_kernel  the same step with the reference's cold-started method
   roofline      the dominant kernel (the warm-started ascent, CAPE only) against
@@ -544,7 +545,7 @@ def pmc_summary(fetch_dir, write_dir, out, ncol, fast_math):
         'warm_ascent': lambda n: 'warm_ascent_kernel<true, true, true, false, false>' in n,
     }
     res = {'ncol': ncol, 'fast_math': fast_math,
-           'kernels': {'plain': 'cape_grid_kernel<float, unsigned int, true, true, false, false>',
+           'kernels': {'plain': 'cape_grid_kernel<float, unsigned int, true, true, false, false, 0>',
                        'warm': 'warm_setup_kernel<true, true, true, false> + '
                                'warm_ascent_kernel<true, true, true, false, false>'}}
     gib = float(1 << 30)
@@ -770,6 +771,36 @@ def timed_interleaved(fns, steps, warmup, stream):
     return {k: sum(a.elapsed_time(b) for a, b in v) / len(v) for k, v in ev.items()}
 
 
+def accuracy_summary(acc):
+    """The headline numbers of an accuracy section: the worst CAPE and CIN
+    errors against the checker on the sample, and against the reference on the
+    columns of the CPU baseline."""
+    out = {k: {x: acc[k][x] for x in ('max_abs_err', 'frac_within_tol')} for k in ('cape', 'cin')}
+    out['columns'] = acc['columns']
+    out['mulev_frac_equal'] = acc['mulev']['frac_equal']
+    out['srh_max_abs_err'] = acc['srh']['max_abs_err']
+    ref = acc.get('vs_reference_cpu_sample')
+    if ref:
+        out['vs_reference'] = {'columns': ref['columns'],
+                               'cape_outside_tol': ref['cape']['outside_tol'],
+                               'cape_max_abs_err': ref['cape']['max_abs_err'],
+                               'cin_outside_tol': ref['cin']['outside_tol'],
+                               'ill_conditioned': ref['outside_tol_columns']['ill_conditioned']}
+    return out
+
+
+def configs_summary(configs, rag):
+    """{workload: {method: ms}} of the other workloads' sections."""
+    out = {}
+    for name, c in (configs or {}).items():
+        for key, sec in ({name: c} if 'plain' in c else
+                         {f'{name}_{k}': v for k, v in c.items()}).items():
+            out[key] = {m: sec[m]['ms'] for m in ('plain', 'warm')}
+    if rag:
+        out['ragged_200k'] = {m: rag[m]['ms'] for m in ('plain', 'warm')}
+    return out
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument('--gpus', type=int, default=1)
@@ -797,6 +828,7 @@ def main():
     ap.add_argument('--pmc-summary', nargs=2, metavar=('FETCH_DIR', 'WRITE_DIR'),
                     help='summarise two rocprofv3 counter runs of --profile-pass')
     ap.add_argument('--pmc-out', default=PMC_FILE)
+    ap.add_argument('--detail', metavar='FILE', help='write the result with every section in full')
     ap.add_argument('--host-only', action='store_true',
                     help='only the host-array (PCIe-inclusive) section, for traces')
     args = ap.parse_args()
@@ -961,7 +993,7 @@ def main():
             [x[sel].cpu().numpy() for x in outs_p[:4]], ref, at(ofn, idx),
             lambda j, k: lfn(int(idx[j]), k))
         del host
-        log(f"[bench] vs reference: {acc['vs_reference_cpu_sample']}")
+        log(f"[bench] vs reference: {accuracy_summary(acc)['vs_reference']}")
     del a, inp
 
     line = {
@@ -996,19 +1028,21 @@ def main():
                      'ops_executed_per_launch': ops_exec,
                      'achieved_executed': ops_exec / (ms_dom / 1e3) / 1e12,
                      'hbm_gbs_algorithmic': bytes_per_column(NLEV) * value / 1e9},
-        'plain_kernel': {'value': ncol / (ms_plain / 1e3), 'ms_per_step': ms_plain,
-                         'accuracy': acc_plain},
+        'plain_kernel': {'value': ncol / (ms_plain / 1e3), 'ms_per_step': ms_plain},
         'speedup_vs_plain': ms_plain / ms,
         'attribution_cape_only_ms': ms_cape,
         'srh_only_ms': ms_srh,
-        'kernel_counts': counts,
-        'surrogate': sur,
-        'accuracy': acc,
-        'configs': configs,
-        'ragged_200k': rag,
+        'accuracy': accuracy_summary(acc),
+        'configs_ms': configs_summary(configs, rag),
         'host_arrays_pcie_inclusive': host_path,
         'cpu_baseline': cpu,
     }
+    # the sections in full go to a file of their own: with them the result line
+    # is longer than what is kept of a run's output
+    if args.detail:
+        with open(args.detail, 'w') as f:
+            json.dump(dict(line, accuracy=acc, accuracy_plain=acc_plain, kernel_counts=counts,
+                           surrogate=sur, configs=configs, ragged_200k=rag), f, indent=1)
     emit(line)
 
 
