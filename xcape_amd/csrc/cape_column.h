@@ -296,13 +296,13 @@ XC_HD __forceinline__ void fp_eval(T p2, T pi2, T logp, T t1, T th1, T qv1, T ql
         fp_eval_raw<ICE, PSEUDO, REG_MIXED>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast,
                                             th2, t2, qv2, ql2, qi2, arg);
         if (__builtin_expect(!arg_small(arg), 0))
-            fp_eval_ops<T, MATH_LIB, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt,
-                                                  thlast, th2, t2, qv2, ql2, qi2);
+            fp_eval_ops<T, MATH_LIB, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast,
+                                          th2, t2, qv2, ql2, qi2);
         return;
     }
 #endif
-    fp_eval_ops<T, MATH, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast, th2,
-                                      t2, qv2, ql2, qi2);
+    fp_eval_ops<T, MATH, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast, th2, t2, qv2,
+                              ql2, qi2);
 }
 
 // Moist-adiabat fixed point for one sub-step from the cold start (:428-480),
@@ -317,8 +317,8 @@ XC_HD __forceinline__ bool solve_substep_ops(T p2, T pi2, T logp, T t1, T th1, T
     int i = 0;
     while (true) {
         i = i + 1;
-        fp_eval_ops<T, MATH, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast, th2,
-                                          t2, qv2, ql2, qi2);
+        fp_eval_ops<T, MATH, ICE>(p2, pi2, logp, t1, th1, qv1, ql1, qi1, qt, thlast, th2, t2,
+                                  qv2, ql2, qi2);
         st.iterations++;
         if (i > 100) return false;
         const T d = th2 - thlast;

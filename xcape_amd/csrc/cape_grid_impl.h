@@ -186,10 +186,11 @@ namespace XC_NS {
 // separate instantiation, so that the counters do not occupy registers in
 // the timed kernels).  LEVELS: also the LFC and EL (a.p_lfc, a.p_el).
 // LOOP: solve_raw's; LOOP_FEW (small launches, see few_columns) also puts `cpw`
-// columns to a wave, the lanes beyond them on its columns again.  (Waves with few lanes switched on run
-// slowly: with fewer than about 12 the same instructions took up to three
-// times as many cycles, so 4096 columns at 4 to a wave took 1.6 ms with the
-// other lanes off and 0.57 ms with them repeating columns.)
+// columns to a wave, the lanes beyond them on its columns again.  (Waves with
+// few lanes switched on run slowly: with fewer than about 12 the same
+// instructions took up to three times as many cycles, so 4096 columns at 4 to a
+// wave took 1.6 ms with the other lanes off and 0.57 ms with them repeating
+// columns.)
 template <typename T, typename IDX, bool ICE, bool PSEUDO, bool STATS, bool LEVELS = false,
           int LOOP = LOOP_LARGE>
 __global__ void __launch_bounds__(256) cape_grid_kernel(CapeGridArgs a, int cpw)
@@ -427,7 +428,6 @@ warm_setup_kernel(CapeGridArgs a)
 // per cpw columns); the lanes draw from that block as they finish their
 // columns, and lane l >= cpw repeats lane l % cpw's.
 constexpr uint32_t WORK_PARTS = 8;
-
 
 __device__ __forceinline__ uint32_t work_part_begin(uint32_t ncol, uint32_t part,
                                                     uint32_t parts)

@@ -111,7 +111,7 @@ struct TrainLds {
     float b2[H], w3[H], red[4][H];
 };
 
-// gelu_f and gelu_grad_f of one argument
+// gelu_f of one argument, and its derivative
 __device__ __forceinline__ void gelu_both(float z, float &h, float &slope)
 {
     const float c = 0.7978845608028654f, a = 0.044715f;

@@ -59,7 +59,7 @@ __host__ __device__ __forceinline__ float bf16_round(float f)
     return r;
 }
 
-// tanh-form GELU and its derivative, FP32: 0.5 z (1 + tanh(c (z + a z^3))).
+// tanh-form GELU, FP32: 0.5 z (1 + tanh(c (z + a z^3))).
 // tanh(u) = 1 - 2 / (1 + exp(2u)), with the hardware exp and reciprocal
 // (about 1 ulp, far below the BF16 rounding of the activations); saturates
 // cleanly for large |u| (the reciprocal of inf is 0).
@@ -70,14 +70,6 @@ __device__ __forceinline__ float gelu_f(float z)
     const float e = __expf(2.0f * u);
     const float t = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
     return 0.5f * z * (1.0f + t);
-}
-__device__ __forceinline__ float gelu_grad_f(float z)
-{
-    const float c = 0.7978845608028654f, a = 0.044715f;
-    const float u = c * (z + a * z * z * z);
-    const float e = __expf(2.0f * u);
-    const float t = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
-    return 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * c * (1.0f + 3.0f * a * z * z);
 }
 
 typedef __bf16 xc_bf16x8 __attribute__((ext_vector_type(8)));

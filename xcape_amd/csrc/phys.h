@@ -192,8 +192,9 @@ __device__ __forceinline__ float pow_core(float x, float y)
 // reciprocal, two Newton steps, one correction by the exact residual) without
 // its operand scaling and special-value fix-up: the same quotient bit for bit
 // wherever that scaling is the identity (a, b and a/b normal, |b| far from
-// overflow); a zero, infinite or NaN operand gives NaN.  Callers re-evaluate
-// with IEEE division when their result is not finite.
+// overflow); a zero, infinite or NaN operand gives NaN.  Callers take IEEE
+// division, or hand the column to one that does, when their result is not
+// finite.
 __device__ __forceinline__ double ddiv_raw(double a, double b)
 {
     double y = __builtin_amdgcn_rcp(b);

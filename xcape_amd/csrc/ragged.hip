@@ -73,7 +73,8 @@ struct StageArgs {
 // 16 rows are in flight together, and the next array's while this one's are
 // written.  Levels above the tallest of the 64 columns (columns of a segment
 // and source are sorted by height) are neither read nor written.  200 000
-// columns of 30 to 137 levels (a copy of their bytes: 73 us): 346 us with the look-ups at each row, 82 so.
+// columns of 30 to 137 levels (a copy of their bytes: 73 us): 346 us with the
+// look-ups at each row, 82 so.
 __global__ void __launch_bounds__(256) stage_kernel(StageArgs a)
 {
     constexpr int ROWS = STAGE_TILE / 4;

@@ -25,11 +25,12 @@
 // A lane per column over transposed copies, with the whole chain in one walk,
 // took for 1024 x 512 columns of 137 levels 490 us for the copies and 4 x 240
 // us for the walks, which waited for their own chains of FP64 operations (one
-// VALU instruction in 24 cycles per wave); this takes 716 us for the call.  It
-// fetches its profiles 2.6 times (3.9 GB): a window is part of a cache line,
-// and the columns in flight are more than the L2 keeps.  Windows of whole
-// lines fetched them 1.0 to 1.6 times and were slower: more levels computed
-// past the outputs' (32 levels to a window), or too few columns in flight.
+// VALU instruction in 24 cycles per wave); this takes 713 us for the call, at
+// one VALU instruction in 6.6 cycles per SIMD.  It fetches 5.05 GB for 1.45 of
+// profiles (read requests, all of 128 bytes): a window is part of a cache
+// line, and the columns in flight are more than the L2 keeps.  Windows of
+// whole lines fetched less and were slower: more levels computed past the
+// outputs' (32 levels to a window), or too few columns in flight.
 #pragma once
 #include "cape_launch.h"
 #include "srh_column.h"
