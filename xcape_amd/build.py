@@ -38,7 +38,9 @@ UNITS = {
     'cape_accurate.hip': ['-ffp-contract=off', '-mllvm', '-amdgpu-mfma-vgpr-form=1',
                           '-falign-loops=64'],
     'cape_fast.hip': ['-ffp-contract=fast-honor-pragmas', '-mllvm', '-amdgpu-mfma-vgpr-form=1'],
-    'ragged.hip': ['-ffp-contract=off'],
+    # (aligned as above: 160 000 mixed columns, plain, 3073 us against 3170 without,
+    # 1000 columns 2253 against 2315)
+    'ragged.hip': ['-ffp-contract=off', '-falign-loops=64'],
     'mlp.hip': ['-ffp-contract=fast'],
     'surrogate_log.hip': ['-ffp-contract=off'],
     'transpose.hip': ['-ffp-contract=off'],
