@@ -773,7 +773,7 @@ def timed_interleaved(fns, steps, warmup, stream):
 
 def accuracy_summary(acc):
     """The headline numbers of an accuracy section: the worst CAPE and CIN
-    errors against the checker on the sample, and against the reference on the
+    errors against the oracle on the sample, and against the reference on the
     columns of the CPU baseline."""
     out = {k: {x: acc[k][x] for x in ('max_abs_err', 'frac_within_tol')} for k in ('cape', 'cin')}
     out['columns'] = acc['columns']
